@@ -21,6 +21,9 @@
 // output is within 2^-10 sum_k |product| of the exact sum.  The scales are
 // applied once per output: (acc * sx) * sw.
 //
+// Decode batches (M <= 64) and grids of too few such tiles run the kernels of
+// fp8_gemm_small.hip, with the same products and scaling.
+//
 // Tiling.  A 512-thread workgroup (8 waves) computes a 256 x 256 tile of Y;
 // wave w owns the 128 x 64 block (w / 4, w % 4) as 8 x 4 MFMA tiles of
 // 16 x 16 (128 fp32 accumulators per lane).  K advances 128 at a time: the
@@ -62,45 +65,19 @@
 // 3681 us, and the staged rows save another 2 % (3749 against 3835 us).
 #include <algorithm>
 
-#include "kc_common.hpp"
+#include "fp8_gemm.hpp"
 
 namespace {
 
-typedef int32_t i32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef __attribute__((address_space(1))) void global_void;
+using namespace kc::fp8;
 
 constexpr int kThreads = 512;
-constexpr int kBM = 256, kBN = 256, kBK = 128;
+constexpr int kBM = 256, kBN = 256;
 constexpr int kTileBytes = kBM * kBK;            // one operand, one step
 constexpr int kStageBytes = 2 * kTileBytes;      // qx rows then qw rows
 constexpr int kScaleOff = 2 * kStageBytes;       // double buffer: 128 KB
 constexpr int kLdsBytes = kScaleOff + (kBM + kBN) * 4;  // + the tile's sx and sw
 constexpr int kGroupM = 4;
-constexpr int kE8M0One = 127;                    // block scale 2^0
-// instruction classes of __builtin_amdgcn_sched_group_barrier
-constexpr int kSchedMfma = 0x008, kSchedDsRead = 0x100;
-
-__device__ __forceinline__ int swizzle(int row) { return (row >> 1) & 7; }
-
-// One global_load_lds_dwordx4: 16 bytes per lane from `g` into LDS at
-// lds_base + 16 * lane.  Written as inline assembly so that the compiler's
-// LDS-wait bookkeeping does not see it: with such a load in flight the
-// compiler cannot count the ordinary LDS reads and drains them all before
-// every use.  The kernel waits for these loads itself (vmcnt(0) before the
-// barrier that publishes the buffer), and the "memory" clobber keeps LDS
-// reads and writes on their side of it.
-__device__ __forceinline__ void lds_dma16(const void* g, uint32_t lds_base) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_base)
-                 : "memory", "m0");
-}
-
-__device__ __forceinline__ uint32_t lds_address(const uint8_t* p) {
-    return static_cast<uint32_t>(reinterpret_cast<size_t>((lds_void*)p));
-}
 
 // Issue the loads of one operand's 256 x 128-byte step tile into LDS.  Wave
 // w fills rows 32 w .. 32 w + 31 with four 1-KB instructions; lane l of
@@ -125,24 +102,6 @@ __device__ __forceinline__ void load_stage(const int8_t* qx, const int8_t* qw, i
                                            uint8_t* stage, int wave, int lane) {
     load_tile_lds(qx, M, K, m0, k0, stage, wave, lane);
     load_tile_lds(qw, N, K, n0, k0, stage + kTileBytes, wave, lane);
-}
-
-// Operand of the 16-row block at tile row r0: lane (i, kb) gets bytes
-// 32 kb .. 32 kb + 31 of row r0 + i; with kvalid < 128 the 16-byte halves at
-// or past kvalid read as zeros.
-template <bool TAIL>
-__device__ __forceinline__ i32x8 read_operand(const uint8_t* tile, int r0, int lane, int kvalid) {
-    const int row = r0 + (lane & 15), kb = lane >> 4, sw = swizzle(row);
-    const uint8_t* p = tile + row * kBK;
-    u32x4 lo = *reinterpret_cast<const u32x4*>(p + 16 * ((2 * kb) ^ sw));
-    u32x4 hi = *reinterpret_cast<const u32x4*>(p + 16 * ((2 * kb + 1) ^ sw));
-    if constexpr (TAIL) {
-        if (32 * kb >= kvalid) lo = u32x4{0u, 0u, 0u, 0u};
-        if (32 * kb + 16 >= kvalid) hi = u32x4{0u, 0u, 0u, 0u};
-    }
-    return i32x8{static_cast<int32_t>(lo.x), static_cast<int32_t>(lo.y), static_cast<int32_t>(lo.z),
-                 static_cast<int32_t>(lo.w), static_cast<int32_t>(hi.x), static_cast<int32_t>(hi.y),
-                 static_cast<int32_t>(hi.z), static_cast<int32_t>(hi.w)};
 }
 
 template <bool TAIL>
@@ -364,6 +323,8 @@ int gemm_fp8(const char* fn, const int8_t* qx, const float* sx, const int8_t* qw
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: null device pointer", fn);
     if (!kc::aligned(qx, 16) || !kc::aligned(qw, 16))
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: qx and qw must be 16-byte aligned", fn);
+    int st = KC_SUCCESS;
+    if (kc::fp8::gemm_small<YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream, &st)) return st;
     const int64_t tm = (M + kBM - 1) / kBM, tn = (N + kBN - 1) / kBN;
     if (tm * tn > INT32_MAX)
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: too many tiles", fn);
