@@ -22,10 +22,12 @@
 // its MFMA sum C is folded into the fp32 accumulator as
 //     acc += s * C + c2 * sum_k X[m, k],   c2 = -s * (136 + z)
 // which removes the +128 encoding offset, the +8 of q ^ 8 and the zero point
-// exactly as the GEMV does.  Groups smaller than 128 fall back to the GEMV
-// per activation row.
+// exactly as the GEMV does.  Groups of 64 and 32 on 16-byte aligned operands
+// run gemm_int4_skinny_kernel, other shapes the GEMV per activation row.
 //
-// Kernels, by M (kc_gemm_int4_bf16 at the bottom picks one):
+// Kernels, by M (kc_gemm_int4_bf16 at the bottom picks one), for more than 8192
+// weight rows (16384 at M <= 16); fewer run gemm_int4_skinny_kernel
+// (int4_gemm_skinny.hip):
 //   M 2..64   gemm_int4_kslds_kernel: K split over the four waves of a CU, X
 //             and the weights streamed into LDS by direct-to-LDS loads; on
 //             the reference layout at M <= 48 with K a multiple of 1024 the
@@ -59,6 +61,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "int4_gemm.hpp"
 #include "kc_common.hpp"
 
 namespace {
@@ -2069,6 +2072,15 @@ int gemm_int4(const char* fn, const uint8_t* d_packed, const float* d_scales,
             if (st >= 0) return st;  // else the X-resident kernel below, at M = 1
         }
     } else if (!fast || m == 1) {
+        // Groups of 64 and 32 from M = 3 on the matrix cores (N 28672, K 4096:
+        // M 3 37.7 -> 25.0 us with groups of 64, 38.7 -> 36.9 with 32; at M 2 the
+        // two GEMVs are as fast or faster, 27.4 against 38.4 us with 32).
+        if (m > 2 && cols > 0 && cols % kTBlock == 0 && (group_size == 64 || group_size == 32) &&
+            kc::aligned(d_packed, 16) && kc::aligned(d_x, 16)) {
+            const int st = kc::int4::gemm_skinny<false>(fn, d_packed, d_scales, d_zeros, d_x, d_y, m, rows, cols,
+                                                        group_size, stream);
+            if (st >= 0) return st;
+        }
         // One GEMV per activation row: same results, no matrix cores (and for
         // a single row the GEMV streams the weights faster: K 8192, N 28672,
         // 20.4 us against 28.3 us for the X-resident kernel below).
@@ -2082,6 +2094,12 @@ int gemm_int4(const char* fn, const uint8_t* d_packed, const float* d_scales,
         return KC_SUCCESS;
     }
     const int gshift = kc::ilog2(group_size) - 7;
+    // Up to N = 8192 (16384 at M <= 16) one or two row tiles per workgroup.
+    {
+        const int st = kc::int4::gemm_skinny<SHUF>(fn, d_packed, d_scales, d_zeros, d_x, d_y, m, rows, cols, group_size,
+                                                   stream);
+        if (st >= 0) return st;
+    }
     // M <= 8 on the reference layout: the K-split kernel below in its pair
     // form where that applies (K a multiple of 1024, up to 12288), else the
     // X-resident kernel when its LDS fits in some number of phases of K.  On

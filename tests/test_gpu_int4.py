@@ -359,6 +359,49 @@ def test_gemm_shapes(gpu, oracle, m, rows, cols, gs):
     assert rel_l2(y, truth) < 3e-3
 
 
+# Few weight rows per workgroup (int4_gemm_skinny.hip): one row tile up to N =
+# 4096, two beyond, one to four tiles of X, ragged N and M at the tile edges,
+# odd T-block counts (the last pair half empty), fewer pairs than waves, groups
+# of several T-blocks, and the groups of 64 and 32 that split a T-block (one
+# group per zero byte and row included).
+SKINNY_SHAPES = [(2, 15, 128, 128), (15, 16, 384, 128), (16, 17, 2048, 256), (17, 4096, 640, 128),
+                 (33, 4097, 1152, 128), (48, 33, 14336, 128), (49, 8192, 256, 256),
+                 (64, 40, 3200, 128), (7, 8193, 1024, 512), (16, 16384, 640, 128),
+                 (2, 1, 128, 64), (3, 1, 128, 64), (16, 31, 640, 64), (17, 4097, 384, 64), (40, 16, 5120, 64),
+                 (64, 8200, 256, 64), (3, 4100, 1152, 32), (15, 48, 128, 32), (33, 100, 640, 32),
+                 (64, 4099, 256, 32)]
+
+
+@pytest.mark.parametrize("m,rows,cols,gs", SKINNY_SHAPES)
+def test_gemm_skinny(gpu, oracle, m, rows, cols, gs):
+    packed, scales, zeros = make_int4(rows, cols, gs, seed=m * 77 + rows)
+    xb = normal_bf16((m, cols), seed=m + cols)
+    y, (dp, ds, dz, dx) = _gemm(gpu, packed, scales, zeros, xb, m, rows, cols, gs)
+    truth = oracle.gemm_int4_bf16_f64(packed, scales, zeros.reshape(-1), xb, m, rows, cols, gs,
+                                      threads=16)
+    for i in range(m):
+        assert rel_l2(y[i], truth[i]) < 3e-3, i
+    if gs >= 128:  # the shuffled layout runs the same products and sums
+        import kernel_craft_torch_ops as ops
+        sh = ops.int4_gemm_bf16_shuffled(ops.int4_shuffle_mfma(dp, rows, cols), ds, dz,
+                                         dx.view(gpu.bfloat16).reshape(m, cols), rows, cols, gs)
+        np.testing.assert_array_equal(bf16_bits_to_f32(_host_bf16_bits(sh)).reshape(m, rows), y)
+
+
+@pytest.mark.parametrize("m,rows,cols,gs", [(4, 16500, 1280, 256), (12, 16400, 24576, 128),
+                                            (40, 8210, 16384, 128), (64, 8200, 24576, 128),
+                                            (20, 8300, 20480, 128)])
+def test_gemm_large_rows(gpu, oracle, m, rows, cols, gs):
+    """More rows than the kernel above takes: X resident in LDS, the chunked
+    fallback, K split with X in registers, the four-tile fallback."""
+    packed, scales, zeros = make_int4(rows, cols, gs, seed=m * 1000 + rows)
+    xb = normal_bf16((m, cols), seed=m + rows)
+    y, _ = _gemm(gpu, packed, scales, zeros, xb, m, rows, cols, gs)
+    truth = oracle.gemm_int4_bf16_f64(packed, scales, zeros.reshape(-1), xb, m, rows, cols, gs,
+                                      threads=16)
+    assert rel_l2(y, truth) < 3e-3
+
+
 # ---------------------------------------------------------------------------
 # A decode step's GEMVs in one launch (kc_gemv_int4_bf16_chain)
 # ---------------------------------------------------------------------------
