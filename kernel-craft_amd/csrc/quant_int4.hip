@@ -592,8 +592,9 @@ __global__ __launch_bounds__(kThreads) void dequant_int4_generic_kernel(
     }
 }
 
-// Fast: 4 packed bytes -> 8 fp32 (two 16-byte stores) per thread; requires
-// K % 8 == 0 and gs % 8 == 0 so the 8 outputs share one group.
+// 4 packed bytes -> 8 fp32 (two 16-byte stores) per thread; requires K % 8 == 0
+// and gs % 8 == 0 so the 8 outputs share one group.  For shapes that the
+// kernel below does not take.
 __global__ __launch_bounds__(kThreads) void dequant_int4_fast_kernel(
     const uint8_t* __restrict__ packed, const float* __restrict__ scales,
     const uint8_t* __restrict__ zeros, float* __restrict__ out, int64_t rows, int64_t cols,
@@ -620,6 +621,60 @@ __global__ __launch_bounds__(kThreads) void dequant_int4_fast_kernel(
         f32x4* o = reinterpret_cast<f32x4*>(out) + 2 * i;
         __builtin_nontemporal_store(lo, o);
         __builtin_nontemporal_store(hi, o + 1);
+    }
+}
+
+// K % 32 == 0 and gs % 32 == 0: a wave takes U runs of 64 chunks (16
+// packed bytes, 32 weights, one group each).  Lane l loads chunk l of a run
+// with its scale and zero point; the run goes through 1 KB of LDS, and store k
+// of 8 writes the 256 outputs of chunks 8 k .. 8 k + 7, lane l the four of
+// halfword l % 8 of chunk 8 k + l / 8, so that each store is 1 KB in address
+// order.  Bound by the writes (8 bytes out per byte in): 14336 x 4096, groups of
+// 128, 71.4 us with two interleaved 16-byte stores per lane and a 64-bit
+// division per 8 weights -> 46.6 us here with U = 4 (266 MB; a fill of the 235 MB
+// written takes 30 us); U = 1 46.4, but 4096 x 4096 14.7 against 12.8.
+template <int U>
+__global__ __launch_bounds__(kThreads) void dequant_int4_chunk_kernel(
+    const uint8_t* __restrict__ packed, const float* __restrict__ scales,
+    const uint8_t* __restrict__ zeros, float* __restrict__ out, uint32_t chunks, uint32_t cpr,
+    uint32_t cpg, uint32_t G) {
+    __shared__ u32x4 run[kWavesPerBlock][U][kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    const uint32_t first = (blockIdx.x * kWavesPerBlock + wave) * (U * kWave);
+    u32x4 w[U];
+    float s[U], zf[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        w[u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(packed) +
+                                          min(first + u * kWave + lane, chunks - 1));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint32_t c = min(first + u * kWave + lane, chunks - 1);
+        const uint32_t row = c / cpr, g = (c - row * cpr) / cpg;
+        s[u] = scales[static_cast<int64_t>(row) * G + g];
+        zf[u] = static_cast<float>(8 + zero_nibble(zeros, row, G, g));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) run[wave][u][lane] = w[u];
+    // this wave's LDS writes before its own reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint16_t* h = reinterpret_cast<const uint16_t*>(run[wave][u]);
+        const uint32_t c0 = first + u * kWave;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int src = 8 * k + (lane >> 3);
+            const float sv = __shfl(s[u], src, kWave), zv = __shfl(zf[u], src, kWave);
+            const uint32_t d = h[64 * k + lane] ^ 0x8888u;  // nibbles n' = q ^ 8 = sext4(q) + 8
+            // n' - (8 + z) is exact, so the product is the only rounding
+            const f32x4 v{(static_cast<float>(d & 0xFu) - zv) * sv, (static_cast<float>((d >> 4) & 0xFu) - zv) * sv,
+                          (static_cast<float>((d >> 8) & 0xFu) - zv) * sv, (static_cast<float>(d >> 12) - zv) * sv};
+            if (c0 + src < chunks)
+                __builtin_nontemporal_store(v, reinterpret_cast<f32x4*>(out) + static_cast<int64_t>(c0) * 8 + 64 * k + lane);
+        }
     }
 }
 
@@ -820,6 +875,19 @@ int dequant_int4(const char* fn, const uint8_t* packed, const float* scales, con
     int st = check_int4_args(fn, packed, scales, zeros, packed, out, rows, cols, gs);
     if (st != KC_SUCCESS) return st;
     if (rows == 0 || cols == 0) return KC_SUCCESS;
+    const int64_t chunks = rows * (cols >> 5);
+    if (cols % 32 == 0 && gs % 32 == 0 && kc::aligned(packed, 16) && kc::aligned(out, 16) && chunks < INT32_MAX) {
+        // four runs per wave where that leaves two workgroups per CU
+        constexpr int64_t kRun = kWavesPerBlock * kWave;
+        const auto launch = [&](auto kernel, int64_t per_block) {
+            kernel<<<static_cast<unsigned>((chunks + per_block - 1) / per_block), kThreads, 0, stream>>>(
+                packed, scales, zeros, out, static_cast<uint32_t>(chunks), static_cast<uint32_t>(cols >> 5),
+                static_cast<uint32_t>(gs >> 5), static_cast<uint32_t>(cols / gs));
+        };
+        if (chunks >= 512 * 4 * kRun) launch(dequant_int4_chunk_kernel<4>, 4 * kRun);
+        else launch(dequant_int4_chunk_kernel<1>, kRun);
+        return kc::check_launch(fn);
+    }
     const bool fast = cols % 8 == 0 && gs % 8 == 0 && kc::aligned(packed, 4) &&
                       kc::aligned(out, 16);
     const int64_t work = fast ? rows * (cols >> 3) : rows * (cols >> 1);

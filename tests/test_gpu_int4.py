@@ -127,6 +127,20 @@ def test_gemv_f32_shapes(gpu, oracle, rows, cols, gs):
     assert rel_l2(y, truth) < TOL_F32
 
 
+# Dequantization in runs of 64 chunks of 32 weights: one and four runs per
+# wave (four from 2^19 chunks), a last run cut anywhere, groups that are not a
+# power of two, one group per row; K and groups not multiples of 32 take the
+# other two kernels.
+@pytest.mark.parametrize("rows,cols,gs", [(1, 32, 32), (65, 32, 32), (3, 1056, 96), (129, 2080, 32),
+                                          (4096, 4096, 128), (4097, 4128, 32), (2731, 6144, 6144),
+                                          (7, 1000, 8), (33, 1032, 24)])
+def test_dequant_runs_bit_exact(gpu, oracle, rows, cols, gs):
+    packed, scales, zeros = make_int4(rows, cols, gs, seed=rows * 3 + cols)
+    out = _dequant(gpu, packed, scales, zeros, rows, cols, gs)
+    exp = oracle.dequantize_int4(packed, scales, zeros.reshape(-1), rows, cols, gs)
+    np.testing.assert_array_equal(out, exp)
+
+
 # Staged-kernel variants: 4 rows per wave (K = 4096 from N = 4096, K = 8192
 # from N = 8192; ragged N, 16- and 64-lane slot maps) and x beyond 64 KB of
 # LDS (fp32 x at K > 15872, up to the 160 KB of K = 32768).
