@@ -381,6 +381,24 @@ def test_e4m3_conversion_exhaustive(gpu, oracle):
         assert bad == 0, f"{bad} mismatches from 0x{start:08x}, first 0x{first:08x}"
 
 
+@pytest.mark.parametrize("per_token", [True, False])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (3, 1020), (2, 1028), (3, 2048), (2, 2052), (5, 4100),
+                                       (7, 1001), (2, 2049)])
+def test_dequant_column_tiles(gpu, oracle, rows, cols, per_token):
+    """One and two 1024-column loads per thread, tiles cut at and beside their
+    edges, and columns that are not a multiple of 4."""
+    torch = gpu
+    rng = np.random.default_rng(rows * 17 + cols)
+    q = rng.integers(-128, 128, (rows, cols)).astype(np.int8)
+    s = rng.uniform(1e-3, 3.0, rows if per_token else 1).astype(np.float32)
+    dq, ds = _dev(torch, q), _dev(torch, s)
+    out = torch.full((rows, cols), 7.0, device="cuda")
+    L = kc_abi.lib()
+    L.launch_dequantize_fp8(ptr(dq), ptr(ds), ptr(out), rows, cols, per_token, stream())
+    kc_abi.check("launch_dequantize_fp8")
+    np.testing.assert_array_equal(out.cpu().numpy(), oracle.dequantize_fp8(q, s, rows, cols, per_token))
+
+
 def test_dequant_all_codes(gpu, oracle):
     torch = gpu
     q = np.tile(np.arange(256, dtype=np.uint8), 8).view(np.int8).reshape(4, 512)
