@@ -212,11 +212,41 @@ def _set(span: Any, key: str, value: Any) -> None:
         pass
 
 
-@contextlib.contextmanager
-def kernel_span(name: str, **attrs: Any) -> Iterator[Any]:
+class _UnrecordedSpan(contextlib.ContextDecorator):
+    """A LocalTracer span opened while nothing records: no attributes to keep
+    and no device time to take (0.5 us of host time per call against 1.6 through
+    the two generators of the recorded form)."""
+
+    __slots__ = ("_name", "_attrs", "_span")
+
+    def __init__(self, name: str, attrs: dict) -> None:
+        self._name = name
+        self._attrs = attrs
+
+    def _recreate_cm(self) -> Any:  # a decorated function decides at each call
+        return kernel_span(self._name, **self._attrs)
+
+    def __enter__(self) -> LocalSpan:
+        self._span = LocalSpan(self._name, recorded=False)
+        return self._span
+
+    def __exit__(self, *exc: Any) -> None:
+        self._span.end_ns = time.perf_counter_ns()
+        for sink in _sinks:
+            sink.append(self._span)
+
+
+def kernel_span(name: str, **attrs: Any) -> Any:
     """Span ``name`` with ``attrs`` around the block; a recorded span also
     gets ``kernel.cuda_ms``, the device time of the work the block queued on
     the current stream (events around the block, waited on at its end)."""
+    if not _sinks and type(_get_tracer()) is LocalTracer:
+        return _UnrecordedSpan(name, attrs)
+    return _traced_span(name, attrs)
+
+
+@contextlib.contextmanager
+def _traced_span(name: str, attrs: dict) -> Iterator[Any]:
     with _get_tracer().start_as_current_span(name) as span:
         live = _recording(span)
         if live:

@@ -159,15 +159,17 @@ def _setup_prototypes(lib: ctypes.CDLL) -> None:
 # ---------------------------------------------------------------------------
 
 
-def _stream() -> ctypes.c_void_p:
-    """The current torch stream (a hipStream_t) for the launchers."""
+def _stream() -> int:
+    """The current torch stream of the current device (a hipStream_t) for the
+    launchers: torch.cuda.current_stream().cuda_stream without the Stream
+    object around it (2.7 -> 0.1 us)."""
     import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(-1)
 
 
-def _ptr(t) -> ctypes.c_void_p:
+def _ptr(t) -> int:
     """Device address of a tensor's first element."""
-    return ctypes.c_void_p(t.data_ptr())
+    return t.data_ptr()
 
 
 def _arg(name: str, t, dtypes=None, numel: Optional[int] = None):
@@ -190,7 +192,7 @@ def _arg(name: str, t, dtypes=None, numel: Optional[int] = None):
 def _on_gpu(op: str, *tensors) -> None:
     """ValueError unless every tensor lives on a GPU."""
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise ValueError(f"{op}: a tensor is on {t.device}; kernel_craft ops run on the "
                              "GPU only (there is no CPU fallback)")
 
@@ -217,6 +219,15 @@ def _int4_weights(op: str, packed, scales, zeros, rows: int, cols: int, group_si
     ok = rows > 0 and cols > 0 and group_size > 0
     packed = _arg(f"{op}: packed", packed, torch.uint8, rows * (cols // 2) if ok else None)
     return (packed,) + _int4_meta(op, scales, zeros, rows, cols, group_size)
+
+
+def _vector(rows: int, cols: int, device):
+    """fp32 [rows] for one result per matrix row.  The kernels write every
+    element of their outputs, so outputs are not cleared first (a fill is a
+    pass of its own: 35 us of device time for 14336 x 4096 fp32).  Rows without
+    columns keep zeros: the quantizer writes nothing for them."""
+    import torch
+    return (torch.empty if cols else torch.zeros)(rows, dtype=torch.float32, device=device)
 
 
 def _check(name: str, status: Optional[int] = None) -> None:
@@ -314,7 +325,7 @@ def int4_dequantize(packed, scales, zeros, rows: int, cols: int, group_size: int
     packed, scales, zeros = _int4_weights("int4_dequantize", packed, scales, zeros, rows, cols,
                                           group_size)
     _on_gpu("int4_dequantize", packed, scales, zeros)
-    out = torch.zeros(rows, cols, dtype=torch.float32, device=packed.device)
+    out = torch.empty(rows, cols, dtype=torch.float32, device=packed.device)
     _get_lib().launch_dequantize_int4(_ptr(packed), _ptr(scales), _ptr(zeros), _ptr(out),
                                       rows, cols, group_size, _stream())
     _check("int4_dequantize")
@@ -329,7 +340,7 @@ def int4_gemv(packed, scales, zeros, x, rows: int, cols: int, group_size: int = 
                                           group_size)
     x = _arg("int4_gemv: x", x, torch.float32, cols)
     _on_gpu("int4_gemv", packed, scales, zeros, x)
-    y = torch.zeros(rows, dtype=torch.float32, device=packed.device)
+    y = _vector(rows, cols, packed.device)
     with kernel_span("int4_gemv", rows=rows, cols=cols, group_size=group_size):
         _get_lib().launch_gemv_int4(_ptr(packed), _ptr(scales), _ptr(zeros), _ptr(x), _ptr(y),
                                     rows, cols, group_size, _stream())
@@ -348,8 +359,9 @@ def fp8_quantize(x, per_token: bool = True) -> Tuple:
     x = _arg("fp8_quantize: x", x, torch.float32)
     _on_gpu("fp8_quantize", x)
     rows, cols = x.shape
-    q = torch.zeros(rows, cols, dtype=torch.int8, device=x.device)
-    scales = torch.zeros(rows if per_token else 1, dtype=torch.float32, device=x.device)
+    q = torch.empty(rows, cols, dtype=torch.int8, device=x.device)
+    scales = _vector(rows, cols, x.device) if per_token else torch.zeros(
+        1, dtype=torch.float32, device=x.device)
     with kernel_span("fp8_quantize", rows=rows, cols=cols, per_token=per_token):
         _get_lib().launch_quantize_fp8(_ptr(x), _ptr(q), _ptr(scales), rows, cols, per_token,
                                        _stream())
@@ -367,7 +379,7 @@ def fp8_dequantize(q, scales, rows: int, cols: int, per_token: bool = True):
     if not per_token and scales.numel() < 1:
         raise ValueError("fp8_dequantize: per-tensor mode needs one scale")
     _on_gpu("fp8_dequantize", q, scales)
-    out = torch.zeros(rows, cols, dtype=torch.float32, device=q.device)
+    out = torch.empty(rows, cols, dtype=torch.float32, device=q.device)
     _get_lib().launch_dequantize_fp8(_ptr(q), _ptr(scales), _ptr(out), rows, cols, per_token,
                                      _stream())
     _check("fp8_dequantize")
@@ -386,7 +398,7 @@ def smoothquant_scale(x, smooth_scales):
     rows, cols = x.shape
     smooth_scales = _arg("smoothquant_scale: smooth_scales", smooth_scales, torch.float32, cols)
     _on_gpu("smoothquant_scale", x, smooth_scales)
-    out = torch.zeros(rows, cols, dtype=torch.float32, device=x.device)
+    out = torch.empty(rows, cols, dtype=torch.float32, device=x.device)
     _get_lib().launch_smoothquant_scale(_ptr(x), _ptr(smooth_scales), _ptr(out), rows, cols,
                                         _stream())
     _check("smoothquant_scale")

@@ -185,6 +185,27 @@ def test_otel_local_spans_record_only_inside_a_recorder():
     otel.setup_tracing()   # no-op without opentelemetry; must not raise
 
 
+def test_otel_unrecorded_span_decides_at_each_use():
+    """A span opened while nothing records reaches a recorder opened inside
+    its block, and a decorated function is recorded when its call is."""
+    import kernel_craft_otel as otel
+    if otel._HAS_OTEL_API:
+        pytest.skip("opentelemetry-api is installed: spans come from OTEL")
+
+    @otel.kernel_span("decorated", rows=3)
+    def work():
+        return 5
+
+    assert work() == 5
+    recorder = otel.recorded_spans()
+    with otel.kernel_span("outer", rows=1):
+        spans = recorder.__enter__()
+        assert work() == 5
+    recorder.__exit__(None, None, None)
+    assert [s.name for s in spans] == ["decorated", "outer"]
+    assert spans[0].attributes == {"rows": 3} and spans[1].attributes == {}
+
+
 def test_otel_timer_skips_capture_and_missing_gpu(monkeypatch):
     """Device timing is never attempted while the stream is being captured
     into a graph, nor without a visible GPU."""

@@ -137,6 +137,41 @@ def test_spans_emitted_with_reference_attributes(gpu):
         assert span.attributes[otel.CUDA_MS_ATTR] >= 0.0
 
 
+@pytest.mark.parametrize("rows,cols", [(3, 64), (5, 100), (257, 4104)])
+def test_outputs_on_reused_memory(gpu, rows, cols):
+    """Outputs are not cleared before a call: on memory that held NaN, and on
+    a side stream, every element is the one computed on fresh memory."""
+    torch = gpu
+    gs = 4
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    packed = torch.randint(0, 256, (rows, cols // 2), dtype=torch.uint8, device="cuda", generator=g)
+    zeros = torch.randint(0, 256, (rows, cols // gs), dtype=torch.uint8, device="cuda", generator=g)
+    scales = torch.rand(rows, cols // gs, device="cuda", generator=g)
+    x = torch.randn(rows, cols, device="cuda", generator=g)
+
+    def calls():
+        q, s = ops.fp8_quantize(x)
+        return [q, s, ops.fp8_dequantize(q, s, rows, cols), ops.smoothquant_scale(x, x[0].abs() + 1.0),
+                ops.int4_dequantize(packed, scales, zeros, rows, cols, gs),
+                ops.int4_gemv(packed, scales, zeros, x[0], rows, cols, gs)]
+
+    def poison():
+        for n in 2 * [rows * cols * 4, rows * cols, rows * 4]:
+            torch.full((n,), 255, dtype=torch.uint8, device="cuda")
+
+    first = [t.clone() for t in calls()]
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        poison()
+        again = calls()
+    side.synchronize()
+    for a, b in zip(first, again):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    empty_q, empty_s = ops.fp8_quantize(torch.empty(rows, 0, device="cuda"))
+    assert empty_q.shape == (rows, 0) and torch.equal(empty_s, torch.zeros(rows, device="cuda"))
+
+
 def test_unrecorded_spans_do_not_synchronize(gpu):
     """Outside a recorder no event is recorded and the host is not blocked:
     a call queued behind a long device sleep returns before it finishes."""
