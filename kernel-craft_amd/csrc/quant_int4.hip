@@ -768,7 +768,10 @@ bool launch_fast(const GemvArgs& a, int rows, int cols, int gshift, size_t lds, 
 // when each lane holds 2 or 4 whole chunks per row and N is large enough
 // (K = 4096 from N = 4096, K = 8192 from N = 8192) -- measured 4-26 % faster
 // there (gate/up 13.0 -> 11.8 us), and 2-20 % slower at N <= 1024 or with a
-// part-filled chunk (K = 5120, 14336).
+// part-filled chunk (K = 5120, 14336).  fp32 x, whose reads from LDS a row
+// shares with the wave's others, also with 3 chunks (K 4128 .. 6144) from
+// N = 8192: 28672 x 5120 20.4 -> 18.1 us, 11001 x 5120 10.4 -> 9.7, but 2000 x 5120
+// 3.8 -> 5.0; with 4 part-filled chunks 14000 x 7168 14.4 -> 14.8.
 template <int CPL, bool XB, bool YB, bool NORM>
 bool launch_fast_cpl(int slot, const GemvArgs& a, int rows, int cols, int gshift, size_t lds,
                      hipStream_t stream) {
@@ -778,6 +781,12 @@ bool launch_fast_cpl(int slot, const GemvArgs& a, int rows, int cols, int gshift
         const bool four = cols == CPL * 2048 && rows >= CPL * 2048;
         if (four && slot == 16) return launch_fast<4, CPL, 16, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
         if (four) return launch_fast<4, CPL, 64, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
+    }
+    if constexpr (CPL == 3 && !XB) {
+        if (rows >= 8192) {
+            if (slot == 16) return launch_fast<4, CPL, 16, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
+            return launch_fast<4, CPL, 64, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
+        }
     }
     if (slot == 16) return launch_fast<R, CPL, 16, WPB, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
     return launch_fast<R, CPL, 64, WPB, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
@@ -793,10 +802,11 @@ bool launch_xl(const GemvArgs& a, int64_t rows, int64_t cols, int gshift, hipStr
     if (cols % 2048 != 0 || rows > INT32_MAX) return false;
     const int kw = static_cast<int>(cols / 2048);
     if (kw < 2 || kw > 8 || (kw == 2 && rows > 16384)) return false;
-    // fp32 x: 3-18 % faster than the staged kernel up to N = 6144 (cfg0 5.27
-    // -> 5.12 us, K 14336 14.8 -> 12.9, K 16384 16.7 -> 13.8), slower from
-    // N = 14336 (the staged kernel's 4 rows per wave)
-    if (!BF16 && rows >= 8192) return false;
+    // fp32 x against the staged kernel: faster at K 4096 (N 4096 3.7 against 3.95
+    // us) and from K 10240 (N 4096, K 14336 9.7 against 11.0), and on few rows
+    // (N 1024, K 8192 3.5 against 4.4); slower at K 6144 and 8192 from N 4096 (6.1
+    // against 5.0, 7.6 against 6.5), and no faster from N 8000 (K 4096 5.42 against 5.36)
+    if (!BF16 && (rows >= 8192 || (rows >= 4096 && (kw == 3 || kw == 4)))) return false;
     const int r = static_cast<int>(rows), c = static_cast<int>(cols);
     // Eight rows per wave halve the waves and the x loads per weight byte:
     // faster from about 24 MiB of weights (N 4096: K 14336 7.60 -> 7.45 us,

@@ -145,11 +145,15 @@ def test_dequant_runs_bit_exact(gpu, oracle, rows, cols, gs):
 # from N = 8192; ragged N, 16- and 64-lane slot maps) and x beyond 64 KB of
 # LDS (fp32 x at K > 15872, up to the 160 KB of K = 32768).
 # Below N = 8192 with K = 2048 x 2..8 the fp32 GEMV takes the per-lane-x
-# kernel instead (ragged N, groups 32..256).
+# kernel instead (ragged N, groups 32..256), at K 6144 and 8192 below N = 4096.
 F32_STAGED_SHAPES = [(8192, 4096, 32), (8195, 4096, 64), (8192, 8192, 128), (8200, 8192, 32),
                      (8200, 16384, 128), (33, 20480, 64), (9, 32768, 128), (5, 31744, 32),
                      (4096, 4096, 32), (4099, 4096, 64), (8191, 4096, 128), (100, 6144, 64),
-                     (4097, 14336, 128), (17, 8192, 256), (40, 16384, 128)]
+                     (4097, 14336, 128), (17, 8192, 256), (40, 16384, 128),
+                     # three chunks per lane: 4 rows per wave from N = 8192, 2 below
+                     (8192, 4128, 32), (8195, 5120, 64), (8193, 6144, 128), (8191, 5120, 128),
+                     # K 6144 and 8192: staged from N = 4096, x per lane below
+                     (4095, 6144, 128), (4096, 6144, 64), (4097, 8192, 128), (4095, 8192, 32)]
 
 
 @pytest.mark.parametrize("rows,cols,gs", F32_STAGED_SHAPES)
