@@ -206,6 +206,34 @@ def test_otel_unrecorded_span_decides_at_each_use():
     assert spans[0].attributes == {"rows": 3} and spans[1].attributes == {}
 
 
+def test_otel_span_is_judged_when_entered():
+    """A span made before a recorder opens and entered inside it is recorded
+    with its attributes; one made inside a recorder and entered after it is
+    not.  A span is entered once, and an exception passes through it."""
+    import kernel_craft_otel as otel
+    if otel._HAS_OTEL_API:
+        pytest.skip("opentelemetry-api is installed: spans come from OTEL")
+
+    early = otel.kernel_span("early", rows=2)
+    with otel.recorded_spans() as spans:
+        with early as span:
+            assert span.is_recording()
+        late = otel.kernel_span("late", rows=4)
+    assert [(s.name, s.attributes["rows"]) for s in spans] == [("early", 2)]
+    with late as span:
+        assert not span.is_recording() and span.attributes == {}
+    for used in (early, late):
+        with pytest.raises(AttributeError):
+            used.__enter__()
+    with pytest.raises(KeyError):
+        with otel.kernel_span("raises"):
+            raise KeyError
+    with otel.recorded_spans() as spans, pytest.raises(KeyError):
+        with otel.kernel_span("raises"):
+            raise KeyError
+    assert [s.name for s in spans] == ["raises"] and spans[0].end_ns is not None
+
+
 def test_otel_timer_skips_capture_and_missing_gpu(monkeypatch):
     """Device timing is never attempted while the stream is being captured
     into a graph, nor without a visible GPU."""
