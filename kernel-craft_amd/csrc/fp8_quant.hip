@@ -800,8 +800,10 @@ bool try_smooth_persistent(const char* fn, const void* in, const float* smooth, 
         const int64_t nslots = cols / (BF16 ? 8 : 4);
         if (nslots < kThreads || nslots > 4 * kThreads) return false;
         if (S == Smooth::kNone && nslots != 4 * kThreads) return false;
-        const bool full = nslots % kThreads == 0;
         const int64_t nv = (nslots + kThreads - 1) / kThreads;
+        // FULL: every thread has NV slots.  Rows of exactly three (768 slots) have
+        // no instance of their own and run the four-slot one with its checks.
+        const bool full = nslots == nv * kThreads && nv != 3;
         if (nv == 1) *st = launch_smooth<1, BF16, S, true>(fn, in, smooth, out, scales, rows, cols, stream);
         else if (nv == 2 && full) *st = launch_smooth<2, BF16, S, true>(fn, in, smooth, out, scales, rows, cols, stream);
         else if (nv == 2) *st = launch_smooth<2, BF16, S, false>(fn, in, smooth, out, scales, rows, cols, stream);

@@ -166,6 +166,34 @@ def test_smooth_div_f32_shapes(gpu, oracle, rows, cols):
     _assert_codes_equal(q, eq)
 
 
+@pytest.mark.parametrize("dtype,mode,cols", [
+    (d, m, c) for d, m, step in (("bf16", "div", 8), ("bf16", "mul", 8), ("f32", "div", 4))
+    for k in (1, 2, 3, 4) for c in (256 * k * step - step, 256 * k * step, 256 * k * step + step)])
+def test_smooth_rows_of_whole_slot_sets(gpu, oracle, dtype, mode, cols):
+    """Rows of 1 to 4 times 256 16-byte slots, and one slot beside each: codes
+    and scales of every row, and nothing written past the last row.  Rows,
+    factors and codes lie inside larger buffers, so that a kernel which took
+    the rows for longer ones would still stay in them."""
+    torch = gpu
+    rows, over = 5, 4096
+    x, _ = outlier_activations(rows + 2, cols, 0.005, 100.0, seed=cols)
+    sm = np.random.default_rng(cols + 7).uniform(0.05, 30.0, cols + over).astype(np.float32)
+    xb = f32_to_bf16_bits(x) if dtype == "bf16" else x
+    dx = _dev_bf16(torch, xb) if dtype == "bf16" else _dev(torch, x)
+    dsm = _dev(torch, sm)
+    dq = torch.full((rows * cols + over,), 0x55, dtype=torch.int8, device="cuda")
+    ds = torch.full((rows + 1,), 7.0, device="cuda")
+    name = f"kc_quantize_fp8_smooth_{mode}_{dtype}"
+    print(f"{name} rows={rows} cols={cols}", flush=True)
+    kc_abi.check(name, getattr(kc_abi.lib(), name)(ptr(dx), ptr(dsm), ptr(dq), ptr(ds), rows, cols, stream()))
+    ref = oracle.quantize_fp8_smooth_div if mode == "div" else oracle.quantize_fp8_smooth_mul_bf16
+    eq, es = ref(xb[:rows], sm[:cols])
+    q, s = dq.cpu().numpy(), ds.cpu().numpy()
+    np.testing.assert_array_equal(s[:rows].view(np.uint32), es.view(np.uint32))
+    _assert_codes_equal(q[:rows * cols].reshape(rows, cols), eq)
+    assert (q[rows * cols:] == 0x55).all() and s[rows] == 7.0
+
+
 def _special_rows(rng, cols):
     """Rows that leave the smoothing division's fast route, between ordinary
     rows: zeros, -0, NaN, infinities, quotients that overflow, all-tiny rows,
