@@ -217,14 +217,19 @@ int launch_skinny(const char* fn, const int8_t* qx, const float* sx, const int8_
     return kc::check_launch(fn);
 }
 
-// Row tiles per workgroup: the fewest that leave at most one workgroup per
-// CU, since every workgroup reads all of X (M 32, K 4096: N 6144 11.5 us at
-// one tile, 9.1 at two; N 28672 37.5 at one, 27.8 at two, 24.5 at four).  Seven
-// (N 28672 in 256 workgroups) only with three or four tiles of X to share:
-// M 64, K 8192 59.5 -> 51.8 us, but M 32, K 4096 24.5 -> 29.4.  At one tile,
-// eight waves with one tile of X and four with more (M 16, N 4096, K 4096 5.9
-// against 6.8 us; M 32, K 14336 18.1 against 16.9); two steps in flight
-// instead of four where a wave has no more (N 1024, K 1024 5.5 -> 4.4).
+// Row tiles per workgroup: one, two or four, the fewest that leave at most one
+// workgroup per CU, since every workgroup reads all of X (M 32, K 4096: N 6144
+// 11.5 us at one tile, 9.1 at two; N 28672 37.5 at one, 27.8 at two, 24.5 at
+// four); four beyond, two of them on a CU.  Seven with three or four tiles of X
+// to share, while they fill one round of the CUs (N 16385 to 28672): M 64,
+// K 8192 54.0 -> 44.0 us at N 17000, 55.5 -> 44.4 at 20480, 61.5 -> 49.0 at 28672,
+// M 48, K 4096 26.3 -> 24.0, 27.3 -> 24.7, 29.8 -> 29.2 (only where four leave a
+// 257th workgroup or so they gain nothing: N 16400 22.0 -> 23.6, M 64 27.9 -> 26.6);
+// with a second round they lose (M 64, K 8192 62.0 us at four against 80.4 at seven at N 28800, 65.2 against
+// 86.0 at 32768), and with two tiles of X too (M 32, N 28672, K 4096 24.5 against
+// 29.4).  At one tile, eight waves with one tile of X and four with more (M 16,
+// N 4096, K 4096 5.9 against 6.8 us; M 32, K 14336 18.1 against 16.9); two steps
+// in flight instead of four where a wave has no more (N 1024, K 1024 5.5 -> 4.4).
 template <int MT, bool YBF16>
 int skinny(const char* fn, const int8_t* qx, const float* sx, const int8_t* qw, const float* sw, void* y, int M, int N,
            int K, hipStream_t stream) {
@@ -236,7 +241,8 @@ int skinny(const char* fn, const int8_t* qx, const float* sx, const int8_t* qw, 
     }
     if (N <= 2 * kRowsPerTile) return launch_skinny<MT, 2, 8, 2, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream);
     if constexpr (MT >= 3) {
-        if (N > 4 * kRowsPerTile) return launch_skinny<MT, 7, 4, 1, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream);
+        if (N > 4 * kRowsPerTile && N <= 7 * kRowsPerTile)
+            return launch_skinny<MT, 7, 4, 1, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream);
     }
     return launch_skinny<MT, 4, 4, 2, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream);
 }

@@ -127,15 +127,17 @@ def test_random_shapes_bit_exact(gpu, oracle, M, N, K):
         assert np.array_equal(y.view(np.uint32), w.view(np.uint32)), (M, N, K, bf16)
 
 
-# Few tokens (M <= 64): one to four tiles of X, one / two / four / seven weight
-# tiles per workgroup (N up to 4096, 8192, 16384 and past them), odd N, K below
-# one step, with a partial last step, and fewer or more steps than the waves
-# of a workgroup.  Larger M: every tile of the small-grid kernel (32 x 64, 64 x
-# 64, 64 x 128, 128 x 128, 256 x 128) with ragged M and N, and K of fewer, as
-# many and more steps than its LDS buffers.
+# Few tokens (M <= 64): one to four tiles of X, one / two / four weight tiles per
+# workgroup (N up to 4096, 8192 and past it), seven from M 33 at N 16385 to
+# 28672 and four again past it, odd N, K below one step, with a partial last
+# step, and fewer or more steps than the waves of a workgroup.  Larger M: every
+# tile of the small-grid kernel (32 x 64, 64 x 64, 64 x 128, 128 x 128, 256 x
+# 128) with ragged M and N, and K of fewer, as many and more steps than its LDS
+# buffers.
 SMALL_GRIDS = [(1, 1, 16), (8, 15, 128), (9, 17, 144), (16, 33, 1040), (5, 40, 2048), (5, 41, 2064),
                (17, 4097, 272), (64, 4096, 1024), (64, 112, 4112), (1, 8200, 2064), (33, 8193, 144),
-               (32, 16400, 400), (48, 16401, 272), (64, 16386, 528)]
+               (32, 16400, 400), (48, 16401, 272), (64, 16386, 528),
+               (33, 28672, 144), (64, 28671, 272), (48, 28673, 272), (64, 32001, 144)]
 SMALL_GRIDS += [(m, n, k) for m, n in ((65, 131), (200, 2704), (500, 2701), (1000, 2700), (1500, 3900))
                 for k in (16, 272, 640, 1168, 2048)]
 
