@@ -770,8 +770,13 @@ bool launch_fast(const GemvArgs& a, int rows, int cols, int gshift, size_t lds, 
 // there (gate/up 13.0 -> 11.8 us), and 2-20 % slower at N <= 1024 or with a
 // part-filled chunk (K = 5120, 14336).  fp32 x, whose reads from LDS a row
 // shares with the wave's others, also with 3 chunks (K 4128 .. 6144) from
-// N = 8192: 28672 x 5120 20.4 -> 18.1 us, 11001 x 5120 10.4 -> 9.7, but 2000 x 5120
-// 3.8 -> 5.0; with 4 part-filled chunks 14000 x 7168 14.4 -> 14.8.
+// N = 16384 (K 5120, groups of 64: 16384 12.8 -> 11.8 us, 28672 20.5 -> 19.0, 50000
+// 34.3 -> 30.3; K 4128 to 6144 and groups of 32 to 128 level to 13 % faster).  A
+// workgroup then takes 16 rows instead of 8, so below that only where the last
+// round of 256 workgroups is not emptier for it: (10240, 12288] and (14336,
+// 16384] (11264 9.57 -> 9.37, 12288 10.2 -> 9.7, 16000 12.4 -> 11.8), but 8200 7.9 ->
+// 8.9, 10240 8.5 -> 9.3, 12600 10.7 -> 11.2; 2000 3.8 -> 5.0.  With 4 part-filled
+// chunks 14000 x 7168 14.4 -> 14.8.
 template <int CPL, bool XB, bool YB, bool NORM>
 bool launch_fast_cpl(int slot, const GemvArgs& a, int rows, int cols, int gshift, size_t lds,
                      hipStream_t stream) {
@@ -783,7 +788,8 @@ bool launch_fast_cpl(int slot, const GemvArgs& a, int rows, int cols, int gshift
         if (four) return launch_fast<4, CPL, 64, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
     }
     if constexpr (CPL == 3 && !XB) {
-        if (rows >= 8192) {
+        const bool same_rounds = (rows + 4095) / 4096 * 2 == (rows + 2047) / 2048;
+        if (rows > 16384 || (rows > 8192 && same_rounds)) {
             if (slot == 16) return launch_fast<4, CPL, 16, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
             return launch_fast<4, CPL, 64, 4, XB, YB, NORM>(a, rows, cols, gshift, lds, stream);
         }

@@ -150,8 +150,11 @@ F32_STAGED_SHAPES = [(8192, 4096, 32), (8195, 4096, 64), (8192, 8192, 128), (820
                      (8200, 16384, 128), (33, 20480, 64), (9, 32768, 128), (5, 31744, 32),
                      (4096, 4096, 32), (4099, 4096, 64), (8191, 4096, 128), (100, 6144, 64),
                      (4097, 14336, 128), (17, 8192, 256), (40, 16384, 128),
-                     # three chunks per lane: 4 rows per wave from N = 8192, 2 below
+                     # three chunks per lane: 2 rows per wave up to N = 10240 and in
+                     # 12289 .. 14336, else 4 (ragged last workgroups of both)
                      (8192, 4128, 32), (8195, 5120, 64), (8193, 6144, 128), (8191, 5120, 128),
+                     (10240, 4160, 64), (10241, 4128, 32), (11001, 5120, 64), (12288, 6144, 128),
+                     (12289, 5120, 128), (14337, 4224, 128), (16387, 5120, 32),
                      # K 6144 and 8192: staged from N = 4096, x per lane below
                      (4095, 6144, 128), (4096, 6144, 64), (4097, 8192, 128), (4095, 8192, 32)]
 
