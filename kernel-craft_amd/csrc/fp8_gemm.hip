@@ -323,11 +323,11 @@ int gemm_fp8(const char* fn, const int8_t* qx, const float* sx, const int8_t* qw
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: null device pointer", fn);
     if (!kc::aligned(qx, 16) || !kc::aligned(qw, 16))
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: qx and qw must be 16-byte aligned", fn);
-    int st = KC_SUCCESS;
-    if (kc::fp8::gemm_small<YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream, &st)) return st;
     const int64_t tm = (M + kBM - 1) / kBM, tn = (N + kBN - 1) / kBN;
     if (tm * tn > INT32_MAX)
         return kc::set_error(KC_ERR_INVALID_ARGUMENT, "%s: too many tiles", fn);
+    int st = KC_SUCCESS;
+    if (kc::fp8::gemm_small<YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream, &st)) return st;
     static bool attr_set = [] {
         return hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_fp8_kernel<YBF16>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) == hipSuccess;

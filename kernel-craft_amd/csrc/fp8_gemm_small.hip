@@ -399,7 +399,7 @@ __global__ __launch_bounds__(64 * WGM * WGN * KG) void gemm_fp8_tile_kernel(
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(S::kLoads * (ST - 2)) : "memory");
         const int64_t k0 = static_cast<int64_t>(KG * (it + ST) + kg) * kBK;
         const uint32_t st = __builtin_amdgcn_readfirstlane(lds0 + (it % ST) * S::kStage);
-const uint8_t* rd = buf + ((it + 1) % ST) * S::kStage;
+        const uint8_t* rd = buf + ((it + 1) % ST) * S::kStage;
         // the loads into LDS and the operand reads spread over the MFMAs: a
         // load holds its wave until the memory pipe takes it
         constexpr int kM = TM * TN, kR = TM + TN, kL = kPerM + kPerN;
@@ -539,7 +539,12 @@ int launch_tile(const char* fn, const int8_t* qx, const float* sx, const int8_t*
 
 // Tiles (the 256 x 256 kernel in front), and what a K step of 128 takes when
 // every CU holds one of them, in hundredths of a microsecond (measured).  The
-// least expected time wins: ceil(tiles / 256) rounds of K / 128 steps.  Against
+// least expected time wins: ceil(tiles / 256) rounds of K / 128 steps each, and
+// what a round takes beside them (start, scales, the last barrier and the
+// stores; 3 to 14 us measured, one figure for all tiles, which decides only
+// between few large and many small tiles at short K: M 4096, N 6144 44.0 us at
+// K 1024 in two rounds of 256 x 256, 53.2 in three of 256 x 128, 68.7 against 70.5
+// at K 2048; M 1500, N 14336 43.8 against 48.2 and 70.4 against 65.5).  Against
 // 256 x 256 tiles: M 128, N 4096, K 4096 48.2 -> 8.5 us (32 x 64); M 256, N 4096,
 // K 14336 193 -> 36.5 (64 x 64); M 512, N 4096, K 4096 49.3 -> 18.3 (64 x 128);
 // M 1000, N 4096, K 14336 148 -> 67.5 (128 x 128); M 1000, N 6144, K 4096 55 ->
@@ -548,15 +553,17 @@ struct TileCost {
     int rows_m, rows_n, cost;
 };
 constexpr int kCus = 256;
+constexpr int kRoundCost = 600;
 constexpr TileCost kTiles[] = {{256, 256, 165}, {256, 128, 97}, {128, 128, 60}, {64, 128, 40}, {64, 64, 28}, {32, 64, 18}};
 
-int best_tile(int64_t M, int64_t N) {
+int best_tile(int64_t M, int64_t N, int64_t K) {
+    const int64_t steps = (K + kBK - 1) / kBK;
     int best = 0;
     int64_t least = INT64_MAX;
     for (int i = 0; i < static_cast<int>(sizeof(kTiles) / sizeof(kTiles[0])); ++i) {
         const TileCost& t = kTiles[i];
         const int64_t tiles = ((M + t.rows_m - 1) / t.rows_m) * ((N + t.rows_n - 1) / t.rows_n);
-        const int64_t cost = (tiles + kCus - 1) / kCus * t.cost;
+        const int64_t cost = (tiles + kCus - 1) / kCus * (steps * t.cost + kRoundCost);
         if (cost < least) least = cost, best = i;
     }
     return best;
@@ -582,7 +589,7 @@ bool gemm_small(const char* fn, const int8_t* qx, const float* sx, const int8_t*
         }
         return true;
     }
-    switch (best_tile(M, N)) {
+    switch (best_tile(M, N, K)) {
         case 1: *status = launch_tile<4, 4, 4, 2, 1, 3, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream); return true;
         case 2: *status = launch_tile<4, 2, 2, 4, 1, 4, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream); return true;
         case 3: *status = launch_tile<4, 2, 1, 4, 2, 3, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream); return true;

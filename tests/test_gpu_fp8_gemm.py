@@ -140,12 +140,14 @@ SMALL_GRIDS = [(1, 1, 16), (8, 15, 128), (9, 17, 144), (16, 33, 1040), (5, 40, 2
                (33, 28672, 144), (64, 28671, 272), (48, 28673, 272), (64, 32001, 144)]
 SMALL_GRIDS += [(m, n, k) for m, n in ((65, 131), (200, 2704), (500, 2701), (1000, 2700), (1500, 3900))
                 for k in (16, 272, 640, 1168, 2048)]
+# K of two steps: two rounds of 256 x 256 tiles, not three of smaller ones
+SMALL_GRIDS += [(1500, 14340, 144)]
 
 
 @pytest.mark.parametrize("M,N,K", SMALL_GRIDS)
 def test_small_grids_bit_exact(gpu, oracle, M, N, K):
     """fp32 and bf16 Y on integer-valued codes, bit for bit, where the 256 x
-    256 tiles are not used."""
+    256 tiles are not used, and at the edge of their use."""
     torch = gpu
     rng = np.random.default_rng(M * 13 + N * 7 + K)
     qx, sx, qw, sw, want = _integer_case(rng, oracle, M, N, K)
