@@ -2072,9 +2072,10 @@ int gemm_int4(const char* fn, const uint8_t* d_packed, const float* d_scales,
             if (st >= 0) return st;  // else the X-resident kernel below, at M = 1
         }
     } else if (!fast || m == 1) {
-        // Groups of 64 and 32 from M = 3 on the matrix cores (N 28672, K 4096:
-        // M 3 37.7 -> 25.0 us with groups of 64, 38.7 -> 36.9 with 32; at M 2 the
-        // two GEMVs are as fast or faster, 27.4 against 38.4 us with 32).
+        // Groups of 64 and 32 from M = 3 on the matrix cores, unless the GEMVs are
+        // expected to be faster (N 28672, K 4096: M 3 37.7 -> 25.0 us with groups of
+        // 64, 38.7 -> 36.9 with 32; at M 2 the two GEMVs are as fast or faster, 27.4
+        // against 38.4 us with 32).
         if (m > 2 && cols > 0 && cols % kTBlock == 0 && (group_size == 64 || group_size == 32) &&
             kc::aligned(d_packed, 16) && kc::aligned(d_x, 16)) {
             const int st = kc::int4::gemm_skinny<false>(fn, d_packed, d_scales, d_zeros, d_x, d_y, m, rows, cols,

@@ -356,6 +356,33 @@ int by_tokens(const char* fn, const uint8_t* packed, const float* scales, const 
     }
 }
 
+// Groups of 64 and 32 at few tokens: whether one GEMV per token is expected to
+// be faster, in ns.  A GEMV takes 2 us and its weights at 5.5 bytes per ns
+// (half a byte each; short rows count as 1650 k); the kernel here 2.9 us and, whatever M, a time per k that
+// follows the rows past 8192 (few rows: every workgroup walks all of K alone) and
+// is longer for groups of 32, above all where their coefficients (9 bytes per k)
+// leave one workgroup per CU.  Measured, GEMVs against this kernel: M 3, K 14336,
+// groups of 32: N 1024 10.4 against 21.4 us, N 4096 23.0 / 23.1, N 28672 121 / 173;
+// groups of 64: N 1024 10.1 / 15.9, N 4096 22.1 / 17.0; M 5, N 512, K 14336, groups of
+// 32 15.7 / 21.2, K 4096 11.1 / 7.7.  Of 720 shapes (M 3 to 12, N 256 to 28672, K 512 to
+// 14336) the choice costs more than 3 % on 7, 13 % at most; from M 7 on the GEMVs
+// are never clearly faster.
+bool gemvs_faster(int M, int N, int K, int group_size) {
+    if (M > 6) return false;
+    const bool half = group_size == 32;
+    const int64_t gemv = 2000 + static_cast<int64_t>(N) * std::max(K, 1650) / 11000;
+    int64_t k = K, ps;  // ps per k
+    if (N <= kOneTileRows) {
+        ps = half ? 1260 : 900;
+    } else if (N <= 2 * kOneTileRows) {
+        ps = half ? 2150 : 1550;
+    } else {
+        k = (k + 1023) / 1024 * 1024;  // whole pairs for each of four waves
+        ps = static_cast<int64_t>(N) * (!half ? 205 : 9 * K <= 80 * 1024 ? 290 : 400) / 1000;
+    }
+    return M * gemv < 2900 + k * ps / 1000;
+}
+
 }  // namespace
 
 namespace kc {
@@ -366,6 +393,7 @@ int gemm_skinny(const char* fn, const uint8_t* packed, const float* scales, cons
                 uint16_t* Y, int M, int N, int K, int group_size, hipStream_t stream) {
     if (K > INT32_MAX / 128) return -1;  // 32-bit offsets of 64 rows of X
     if constexpr (!SHUF) {
+        if (group_size < kTBlock && gemvs_faster(M, N, K, group_size)) return -1;
         if (group_size == 64) return by_tokens<2, false>(fn, packed, scales, zeros, X, Y, M, N, K, 0, stream);
         if (group_size == 32) return by_tokens<4, false>(fn, packed, scales, zeros, X, Y, M, N, K, 0, stream);
     }

@@ -409,6 +409,25 @@ def test_gemm_skinny(gpu, oracle, m, rows, cols, gs):
         np.testing.assert_array_equal(bf16_bits_to_f32(_host_bf16_bits(sh)).reshape(m, rows), y)
 
 
+@pytest.mark.parametrize("m,rows,cols,gs", [(2, 4096, 4096, 64), (3, 1000, 14336, 64), (3, 257, 8192, 32),
+                                            (5, 500, 14336, 32), (6, 33, 14336, 32), (4, 16400, 14336, 32)])
+def test_gemm_small_groups_per_row(gpu, oracle, m, rows, cols, gs):
+    """Groups of 64 and 32 where one GEMV per token is faster than the kernel
+    above (two tokens; three to six on few rows or large K): the same bits as
+    kc_gemv_int4_bf16 on each row of X."""
+    torch = gpu
+    packed, scales, zeros = make_int4(rows, cols, gs, seed=m * 5 + rows)
+    xb = normal_bf16((m, cols), seed=m + cols)
+    y, (dp, ds, dz, dx) = _gemm(torch, packed, scales, zeros, xb, m, rows, cols, gs)
+    truth = oracle.gemm_int4_bf16_f64(packed, scales, zeros.reshape(-1), xb, m, rows, cols, gs, threads=16)
+    row = torch.empty(rows, dtype=torch.int16, device="cuda")
+    for i in range(m):
+        assert rel_l2(y[i], truth[i]) < 3e-3, i
+        kc_abi.check("kc_gemv_int4_bf16", kc_abi.lib().kc_gemv_int4_bf16(
+            ptr(dp), ptr(ds), ptr(dz), ptr(dx.reshape(m, cols)[i]), ptr(row), rows, cols, gs, stream()))
+        np.testing.assert_array_equal(bf16_bits_to_f32(row.cpu().numpy().view(np.uint16)), y[i])
+
+
 @pytest.mark.parametrize("m,rows,cols,gs", [(4, 16500, 1280, 256), (12, 16400, 24576, 128),
                                             (40, 8210, 16384, 128), (64, 8200, 24576, 128),
                                             (20, 8300, 20480, 128)])
