@@ -987,14 +987,17 @@ int smoothquant_stats(const char* fn, const void* x, int64_t tokens, const void*
     if (blocks_x + blocks_w > 0) {
         const bool vec_x = cols % (BF16 ? 8 : 4) == 0 && kc::aligned(x, 16);
         const bool vec_w = cols % (BF16 ? 8 : 4) == 0 && kc::aligned(w, 16);
-        // Both tensors fit in the 256 MB Infinity Cache: read so that they stay
-        // there, since the quantizers read them next (statistics and both
-        // quantizers, X 2003 x 4096 and W 14336 x 4096 bf16: 71.9 -> 66.0 us, 700 and
-        // 6000 x 5000 57.9 -> 54.9, 1000 and 4096 x 8192 49.4 -> 46.0; the
-        // statistics by themselves 28.3 -> 30.5, 18.9 -> 18.1 and 18.5 -> 17.7).
-        // Beyond it they would push themselves out, and the statistics of X
-        // 16384 x 8192 and W 28672 x 8192 take 117 us streamed, 127 kept.
-        const bool keep = (tokens + outs) * cols * (BF16 ? 2 : 4) <= int64_t{256} << 20;
+        // Up to 28 MB of X and W, ordinary loads leave them in the Infinity Cache
+        // for the quantizers and cost the statistics nothing (new X and W at each
+        // call, alone / followed by both quantizers: 1000 and 2000 x 4096 bf16 10.2 ->
+        // 9.8 / 23.1 -> 21.9 us, 1000 and 6144 x 2048 11.0 -> 10.7 / 24.6 -> 23.5, 512 and
+        // 1024 x 4096 fp32 9.5 -> 9.1 / 23.5 -> 22.7; level at 2 MB).  Larger ones
+        // are streamed: kept, the quantizers gain 3 to 9 % at any size (2003 and
+        // 14336 x 4096 70.9 -> 65.1), but the statistics by themselves, as a calibration
+        // runs them, lose 4 to 18 % at 38 to 60 MB (512 and 4096 x 4096 12.5 -> 13.0, on
+        // the same tensors 10.2 -> 11.0) and 6 to 10 % on new tensors beyond (28.0 ->
+        // 30.0; 28672 x 8192 85 -> 94).
+        const bool keep = (tokens + outs) * cols * (BF16 ? 2 : 4) <= int64_t{28} << 20;
         const auto kernel = keep ? col_absmax2_kernel<BF16, true> : col_absmax2_kernel<BF16, false>;
         kernel<<<static_cast<unsigned>(blocks_x + blocks_w), kThreads, 0, stream>>>(
             x, amax_x, tokens, vec_x, blocks_x, w, amax_w, outs, vec_w, cols, tiles);

@@ -535,7 +535,9 @@ def test_col_absmax_shapes(gpu, oracle, dtype, rows, cols):
 
 @pytest.mark.parametrize("dtype", ["f32", "bf16"])
 @pytest.mark.parametrize("T,N,D", [(256, 384, 8192), (1, 1, 8), (130, 257, 4104), (300, 7, 20),
-                                   (0, 64, 2048), (64, 0, 2048), (5, 3, 1000)])
+                                   (0, 64, 2048), (64, 0, 2048), (5, 3, 1000),
+                                   # past 28 MB: streamed instead of kept in the cache
+                                   (300, 4000, 4104)])
 def test_smoothquant_stats_one_call(gpu, oracle, dtype, T, N, D):
     """kc_smoothquant_stats_* (both maxima and the factors from one call)
     equals kc_col_absmax_* on X and on W followed by kc_smooth_factors, bit
