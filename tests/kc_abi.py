@@ -41,3 +41,19 @@ def check(name: str, status: int | None = None) -> None:
         code = status
     if code:
         raise RuntimeError(f"{name}: kc_status {code}: {L.kc_last_error_string().decode()}")
+
+
+def kernels_of(call) -> list[str]:
+    """Names of the device kernels that call() launches, as the profiler
+    reports them; skips the test where it reports none at all."""
+    import pytest
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CUDA], acc_events=True) as p:
+        call()
+        torch.cuda.synchronize()
+    names = [e.name for e in p.events() if "CUDA" in str(e.device_type)]
+    if not names:
+        pytest.skip("the profiler reports no kernels here")
+    return names

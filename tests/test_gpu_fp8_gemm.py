@@ -84,9 +84,8 @@ def _integer_case(rng, oracle, M, N, K):
 @pytest.mark.parametrize("bf16", [False, True])
 def test_integer_codes_bit_exact(gpu, oracle, M, N, K, bf16):
     """fp32 Y equals the exact sum scaled as (acc * sx) * sw; bf16 Y is that
-    value rounded to nearest even.  N covers every output path: N % 8 == 0
-    (bf16 rows staged through LDS), N % 4 == 0 (four columns per lane) and
-    the rest (one column at a time)."""
+    value rounded to nearest even.  M <= 64 and the smallest tiles, with N %
+    4 == 0 (four columns per lane), N % 2 == 0 (pairs at M <= 64) and the rest."""
     torch = gpu
     rng = np.random.default_rng(M * 7 + N * 3 + K)
     qx, sx, qw, sw, want = _integer_case(rng, oracle, M, N, K)
@@ -101,9 +100,9 @@ def test_integer_codes_bit_exact(gpu, oracle, M, N, K, bf16):
 
 
 def _random_shapes(n, seed=2024):
-    """Seeded shapes over every output path: N a multiple of 8 (bf16 rows
-    staged through LDS), of 4 (four columns per lane) or neither, with M, N
-    and K tails of every size."""
+    """Seeded shapes of M <= 64 and the smallest tiles: N a multiple of 8, of
+    4 (four columns per lane) or neither, with M, N and K tails of every
+    size."""
     rng = np.random.default_rng(seed)
     out = []
     for i in range(n):
@@ -157,15 +156,56 @@ def test_small_grids_bit_exact(gpu, oracle, M, N, K):
         assert np.array_equal(y.view(np.uint32), w.view(np.uint32)), (M, N, K, bf16)
 
 
+# The 256 x 256 tiles: grids that smaller tiles would take more rounds for.  M
+# and N tails and whole tiles, N a multiple of 8 (bf16 rows staged through LDS),
+# of 4 (four columns per lane) and odd, and K of a partial step only, one whole
+# step, one and a tail, odd and even step counts.
+BIG_TILES = [(2945, 2696, 16), (2945, 2700, 272), (3071, 2689, 128), (3072, 2816, 144), (500, 16520, 640),
+             (512, 16516, 1040), (449, 16641, 400)]
+
+
+@pytest.mark.parametrize("M,N,K", BIG_TILES)
+def test_big_tiles_bit_exact(gpu, oracle, M, N, K):
+    """fp32 and bf16 Y on integer-valued codes, bit for bit, on the 256 x 256
+    tiles."""
+    torch = gpu
+    rng = np.random.default_rng(M * 5 + N * 3 + K)
+    qx, sx, qw, sw, want = _integer_case(rng, oracle, M, N, K)
+    for bf16 in (True, False):
+        y = _gemm(torch, qx, sx, qw, sw, bf16=bf16)
+        w = bf16_bits_to_f32(f32_to_bf16_bits(want)) if bf16 else want
+        assert np.array_equal(y.view(np.uint32), w.view(np.uint32)), (M, N, K, bf16)
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(m, n, k, "gemm_fp8_kernel<") for m, n, k in BIG_TILES + [(1500, 14340, 144)]] + [
+    (64, 4096, 1024, "gemm_fp8_skinny_kernel<4, 1,"), (33, 8193, 144, "gemm_fp8_skinny_kernel<3, 4,"),
+    (64, 28671, 272, "gemm_fp8_skinny_kernel<4, 7,"), (48, 28673, 272, "gemm_fp8_skinny_kernel<3, 4,"),
+    (65, 131, 2048, "gemm_fp8_tile_kernel<2, 2, 1, 2,"), (200, 2704, 16, "gemm_fp8_tile_kernel<4, 2, 1, 2,"),
+    (500, 2701, 16, "gemm_fp8_tile_kernel<4, 2, 1, 4,"), (1000, 2700, 2048, "gemm_fp8_tile_kernel<4, 2, 2, 4,"),
+    (1500, 3900, 2048, "gemm_fp8_tile_kernel<4, 4, 4, 2,")])
+def test_kernel_of_shape(gpu, M, N, K, kernel):
+    """The shapes above run the kernel that they are there for."""
+    torch = gpu
+    q = torch.zeros(max(M, N) * K, dtype=torch.int8, device="cuda")
+    s = torch.ones(max(M, N), device="cuda")
+    y = torch.empty(M * N, dtype=torch.float32, device="cuda")
+    for fn in (kc_abi.lib().kc_gemm_fp8_w8a8_bf16, kc_abi.lib().kc_gemm_fp8_w8a8_f32):
+        names = kc_abi.kernels_of(lambda: kc_abi.check("kc_gemm_fp8_w8a8", fn(
+            ptr(q), ptr(s), ptr(q), ptr(s), ptr(y), M, N, K, stream())))
+        assert len(names) == 1 and kernel in names[0], names
+
+
 @pytest.mark.parametrize("bf16,offset", [(True, 0), (True, 1), (True, 4), (False, 1), (False, 2),
                                           (False, 4)])
-def test_output_alignment(gpu, oracle, bf16, offset):
+@pytest.mark.parametrize("M,N,K", [(200, 256, 272), (2945, 2696, 272), (9, 256, 272)])
+def test_output_alignment(gpu, oracle, bf16, offset, M, N, K):
     """Y at an element offset inside a larger buffer (N % 8 == 0): the
-    16-byte row stores need 16-byte alignment, the four-column stores 8 (bf16)
-    or 16 (fp32) bytes; other offsets take the one-column path.  Bit-exact on
-    integer codes, and nothing outside Y is written."""
+    16-byte row stores of the 256 x 256 tiles need 16-byte alignment, the
+    four-column stores (also those of the smaller tiles, 200 x 256) 8 (bf16) or
+    16 (fp32) bytes, the column pairs of M <= 64 4 bytes; other offsets take
+    the one-column path.  Bit-exact on integer codes, and nothing outside Y is
+    written."""
     torch = gpu
-    M, N, K = 200, 256, 272
     rng = np.random.default_rng(offset * 13 + bf16)
     qx, sx, qw, sw, want = _integer_case(rng, oracle, M, N, K)
     dqx, dsx, dqw, dsw = _dev(torch, qx), _dev(torch, sx), _dev(torch, qw), _dev(torch, sw)
@@ -186,7 +226,7 @@ def test_output_alignment(gpu, oracle, bf16, offset):
     assert np.array_equal(got.view(np.uint16 if bf16 else np.uint32), want.view(np.uint16 if bf16 else np.uint32))
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES)
+@pytest.mark.parametrize("M,N,K", SHAPES + [(2945, 2696, 400)])
 @pytest.mark.parametrize("bf16", [False, True])
 def test_full_range_codes_vs_oracle(gpu, oracle, M, N, K, bf16):
     torch = gpu
