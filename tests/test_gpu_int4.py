@@ -320,56 +320,46 @@ def test_gemm_cfg3(gpu, oracle, m):
 @pytest.mark.parametrize("m,rows,cols,gs", [(1, 100, 1024, 128), (3, 64, 256, 128),
                                             (17, 130, 2048, 256), (33, 48, 640, 128),
                                             (64, 16, 128, 128), (5, 40, 512, 64),
-                                            # M <= 4, X resident in LDS: ragged row
-                                            # tiles, spare waves, odd T-block counts,
-                                            # larger groups
+                                            # all from M = 2 on the kernel for few weight
+                                            # rows (int4_gemm_skinny.hip), M = 1 on the
+                                            # GEMV; one tile of X: ragged row tiles, odd
+                                            # T-block counts, larger groups
                                             (2, 250, 384, 128), (1, 17, 128, 128),
                                             (4, 1000, 1280, 256), (3, 4096, 4096, 128),
                                             (4, 7 * 16 * 3 + 5, 2048, 512),
-                                            # M <= 4 whose X does not fit in LDS
+                                            # more T-block pairs than waves
                                             (4, 33, 32768, 128),
-                                            # M 5..8: X in LDS in one, two and four
-                                            # phases of K; M 9..16 on the K-split
-                                            # kernel, or past its LDS on the chunked one
+                                            # M 5..16, K up to 24576
                                             (16, 48, 1024, 128), (8, 300, 4096, 128),
                                             (12, 257, 2048, 256), (16, 100, 8192, 128),
                                             (6, 7 * 16 + 1, 8192, 512), (8, 500, 8192, 128),
                                             (12, 100, 24576, 128), (9, 40, 2048, 256),
-                                            # M 17..64, K split over four waves:
-                                            # ragged rows and activation tiles,
-                                            # waves with no T-block (K < 512),
-                                            # ranges of unequal length
+                                            # M 17..64, two to four tiles of X: ragged
+                                            # rows and activation tiles, waves with no
+                                            # T-block (K < 2048), ranges of unequal length
                                             (33, 70, 1024, 128), (64, 7 * 16 * 2 + 9, 2048, 256),
                                             (48, 200, 8192, 128), (20, 224, 4096, 128),
                                             (32, 1000, 4096, 128), (40, 113, 16384, 128),
                                             (17, 7, 256, 256), (63, 1, 512, 128),
                                             (26, 130, 1152, 128), (40, 200, 4096, 512),
-                                            # M 33..64 whose coefficients do not fit
-                                            # in LDS: the X-resident fallback
+                                            # a coefficient table of 27 KB
                                             (64, 50, 24576, 128),
-                                            # reference layout in pairs of T-blocks:
-                                            # one pair per wave, three and five pairs
-                                            # with groups of 256 / 512, ragged rows, and
-                                            # K at the pair form's LDS limit for one to
-                                            # four activation tiles; three pairs with a
-                                            # last group of two T-blocks for the
-                                            # zero-point pass
+                                            # K a multiple of 1024: whole pairs of
+                                            # T-blocks, one to six per wave, groups of
+                                            # 256 and 512
                                             (3, 200, 1024, 128), (2, 77, 3072, 256),
                                             (5, 1000, 5120, 512), (8, 130, 12288, 128),
                                             (32, 100, 9216, 128), (20, 60, 10240, 128),
                                             (36, 90, 12288, 128), (64, 100, 8192, 128),
                                             (50, 77, 3072, 256),
-                                            # four activation tiles, one T-block at a
-                                            # time: tiles past the last row, two
-                                            # T-blocks per wave, K at the pair form's
-                                            # limit for one tile fewer
+                                            # four activation tiles, the last one with
+                                            # one or two rows
                                             (50, 80, 3072, 256), (49, 224, 1024, 128),
                                             (64, 96, 8192, 128),
-                                            # the pair form with fewer rows than one
-                                            # 16-row tile (every row clamped to N - 1)
+                                            # fewer rows than one 16-row tile (every row
+                                            # clamped to N - 1)
                                             (9, 5, 2048, 128), (2, 1, 1024, 128),
-                                            # M 33..64 with fewer rows than a workgroup's
-                                            # 112, K 2048-6144
+                                            # M 33..64, K 2048-6144
                                             (40, 40, 2048, 128), (64, 16, 4096, 128),
                                             (35, 200, 6144, 128), (57, 1000, 2048, 128)])
 def test_gemm_shapes(gpu, oracle, m, rows, cols, gs):
@@ -428,18 +418,80 @@ def test_gemm_small_groups_per_row(gpu, oracle, m, rows, cols, gs):
         np.testing.assert_array_equal(bf16_bits_to_f32(row.cpu().numpy().view(np.uint16)), y[i])
 
 
-@pytest.mark.parametrize("m,rows,cols,gs", [(4, 16500, 1280, 256), (12, 16400, 24576, 128),
-                                            (40, 8210, 16384, 128), (64, 8200, 24576, 128),
-                                            (20, 8300, 20480, 128)])
+# More rows than the kernel above takes (N past 16384 at M <= 16, past 8192
+# beyond), with the kernel that the shape is there for.
+LARGE_ROWS = [
+    # K split over four waves, operands through LDS, in pairs of T-blocks (K a
+    # multiple of 1024, one to three tiles of X): ragged rows and tiles, one and
+    # three pairs per wave, groups of 256 to 1024, K at the LDS limit of each
+    ((8, 16401, 3072, 256), "gemm_int4_kslds_kernel<1, false, true>"),
+    ((5, 16500, 12288, 512), "gemm_int4_kslds_kernel<1, false, true>"),
+    ((2, 16385, 1024, 128), "gemm_int4_kslds_kernel<1, false, true>"),
+    ((17, 8300, 2048, 1024), "gemm_int4_kslds_kernel<2, false, true>"),
+    ((32, 8193, 9216, 128), "gemm_int4_kslds_kernel<2, false, true>"),
+    ((48, 8210, 2048, 256), "gemm_int4_kslds_kernel<3, false, true>"),
+    ((40, 8209, 3072, 256), "gemm_int4_kslds_kernel<3, false, true>"),
+    ((36, 8200, 12288, 128), "gemm_int4_kslds_kernel<3, false, true>"),
+    # one T-block at a time: odd counts, fewer than waves, K at the LDS limits
+    ((12, 16401, 1152, 128), "gemm_int4_kslds_kernel<1, false, false>"),
+    ((16, 16390, 16384, 256), "gemm_int4_kslds_kernel<1, false, false>"),
+    ((26, 8210, 1152, 128), "gemm_int4_kslds_kernel<2, false, false>"),
+    ((32, 8195, 13824, 256), "gemm_int4_kslds_kernel<2, false, false>"),
+    ((40, 8195, 1152, 128), "gemm_int4_kslds_kernel<3, false, false>"),
+    ((33, 8201, 11776, 128), "gemm_int4_kslds_kernel<3, false, false>"),
+    ((64, 8201, 3200, 128), "gemm_int4_kslds_kernel<4, false, false>"),
+    ((49, 8193, 9216, 1024), "gemm_int4_kslds_kernel<4, false, false>"),
+    ((64, 8300, 256, 256), "gemm_int4_kslds_kernel<4, false, false>"),
+    # coefficients past that kernel's LDS: the same split through registers
+    ((16, 16400, 17408, 128), "gemm_int4_kslice_kernel<1,"),
+    ((20, 8300, 20480, 128), "gemm_int4_kslice_kernel<2,"),
+    ((40, 8210, 16384, 128), "gemm_int4_kslice_kernel<3,"),
+    ((64, 8200, 10240, 128), "gemm_int4_kslice_kernel<4,"),
+    # X resident in LDS, in one or more phases of K
+    ((4, 16400, 16384, 128), "gemm_int4_xres_kernel<"),
+    ((8, 16400, 16384, 512), "gemm_int4_xres_kernel<"),
+    ((3, 16385, 24576, 256), "gemm_int4_xres_kernel<"),
+    ((12, 16400, 24576, 256), "gemm_int4_xres_kernel<"),
+    # four tiles of X resident
+    ((40, 8200, 24576, 128), "gemm_int4_xbig_kernel<"),
+    ((48, 8195, 23552, 256), "gemm_int4_xbig_kernel<"),
+    # chunks of K through LDS
+    ((4, 16500, 1280, 256), "gemm_int4_mfma_kernel<1,"),
+    ((12, 16400, 24576, 128), "gemm_int4_mfma_kernel<1,"),
+    ((32, 8200, 24576, 128), "gemm_int4_mfma_kernel<2,"),
+    ((40, 8200, 24704, 128), "gemm_int4_mfma_kernel<3,"),
+    ((64, 8200, 24576, 128), "gemm_int4_mfma_kernel<4,"),
+]
+
+
+@pytest.mark.parametrize("m,rows,cols,gs", [shape for shape, _ in LARGE_ROWS])
 def test_gemm_large_rows(gpu, oracle, m, rows, cols, gs):
-    """More rows than the kernel above takes: X resident in LDS, the chunked
-    fallback, K split with X in registers, the four-tile fallback."""
     packed, scales, zeros = make_int4(rows, cols, gs, seed=m * 1000 + rows)
     xb = normal_bf16((m, cols), seed=m + rows)
     y, _ = _gemm(gpu, packed, scales, zeros, xb, m, rows, cols, gs)
     truth = oracle.gemm_int4_bf16_f64(packed, scales, zeros.reshape(-1), xb, m, rows, cols, gs,
                                       threads=16)
-    assert rel_l2(y, truth) < 3e-3
+    for i in range(m):
+        assert rel_l2(y[i], truth[i]) < 3e-3, i
+
+
+@pytest.mark.parametrize("shape,kernel", LARGE_ROWS + [
+    ((16, 16384, 640, 128), "gemm_int4_skinny_kernel<1, 2, 4, 1, false>"),
+    ((16, 4096, 640, 128), "gemm_int4_skinny_kernel<1, 1, 8, 1, false>"),
+    ((64, 8192, 640, 128), "gemm_int4_skinny_kernel<4, 2, 4, 1, false>"),
+    ((64, 8200, 256, 64), "gemm_int4_skinny_kernel<4, 2, 4, 2, false>"),
+    ((3, 4100, 1152, 32), "gemm_int4_skinny_kernel<1, 2, 8, 4, false>")])
+def test_kernel_of_shape(gpu, shape, kernel):
+    """The shapes above run the kernel that they are there for."""
+    torch = gpu
+    m, rows, cols, gs = shape
+    G = cols // gs
+    w, z = (torch.zeros(n, dtype=torch.uint8, device="cuda") for n in (rows * cols // 2, rows * ((G + 1) // 2)))
+    s = torch.ones(rows * G, device="cuda")
+    x, y = (torch.zeros(n, dtype=torch.bfloat16, device="cuda") for n in (m * cols, m * rows))
+    names = kc_abi.kernels_of(lambda: kc_abi.check("kc_gemm_int4_bf16", kc_abi.lib().kc_gemm_int4_bf16(
+        ptr(w), ptr(s), ptr(z), ptr(x), ptr(y), m, rows, cols, gs, stream())))
+    assert len(names) == 1 and kernel in names[0], names
 
 
 # ---------------------------------------------------------------------------
