@@ -227,11 +227,13 @@ int kc_gemm_int4_bf16(const uint8_t* d_packed, const float* d_scales,
  *   kc_shuffle_int4_mfma: packed [rows, cols/2] -> that buffer (16-byte
  *     aligned, not overlapping).
  *   kc_gemm_int4_bf16_shuffled: kc_gemm_int4_bf16 on the shuffled weights,
- *     each wave-wide load reading 1 KB of the layout.  For m >= 9, and for
- *     m 2..8 with rows up to 16384 or cols a multiple of 1024 up to 12288,
- *     the same kernel as kc_gemm_int4_bf16 on the same values: bit-identical
- *     results.  Other m 2..8 shapes run the K-split kernel here and the X-resident kernel
- *     on the reference layout (another summation order).  m == 1 runs a matrix-core GEMV when cols = 1024 * KW (KW <= 16), or
+ *     each wave-wide load reading 1 KB of the layout.  Bit-identical results
+ *     (the same products and sums) with rows up to 16384 at m 2..16 and up
+ *     to 8192 at m 17..64 (cols up to 72704), and with more rows for m >= 9
+ *     except m 33..48 at cols == 12288, and for m 2..8 at cols a multiple of
+ *     1024 up to 12288 or past 23040.  The other shapes run kernels of
+ *     another summation order on the two layouts.  m == 1 runs a matrix-core
+ *     GEMV when cols = 1024 * KW (KW <= 16), or
  *     cols = 512 * KW (KW <= 16) with rows <= 8192 (four k-blocks per wave);
  *     other cols take the m >= 2 kernel.  Within the bf16 tolerance of the
  *     reference GEMV.  Needs cols % 128 == 0, group_size a power of two

@@ -2,14 +2,11 @@
 kc_gemm_int4_bf16_shuffled): the weight-format bridge's optional
 "MFMA-friendly" layout.  Bars: the conversion bit for bit against the oracle
 (kco_shuffle_int4_mfma, itself pinned in test_oracle.py); where both layouts
-run the same kernel (m >= 9, and m 2..8 with K a multiple of 1024 up to
-12288, where the reference layout takes the K-split kernel's pair form) the
-GEMM on the shuffled layout bit for bit against kc_gemm_int4_bf16 on the
-reference layout (the same arithmetic, other addresses); for the other
-m 2..8 shapes (the K-split kernel on the shuffled layout, the X-resident
-kernel on the reference layout: other summation orders) and m == 1 (a
-matrix-core GEMV of its own) within the bf16 tolerance of the fp64 oracle, as
-the other bf16 GEMM and GEMV tests."""
+run the same products and sums (same_sums below: all but some shapes of many
+rows) the GEMM on the shuffled layout bit for bit against kc_gemm_int4_bf16
+on the reference layout; for the others (another summation order) and m == 1
+(a matrix-core GEMV of its own) within the bf16 tolerance of the fp64 oracle,
+as the other bf16 GEMM and GEMV tests."""
 import ctypes
 
 import numpy as np
@@ -18,6 +15,7 @@ import pytest
 import kc_abi
 from kc_abi import ptr, stream
 from kc_data import bf16_bits_to_f32, make_int4, normal_bf16, rel_l2
+from test_gpu_int4 import LARGE_ROWS
 
 pytestmark = pytest.mark.gpu
 
@@ -71,9 +69,10 @@ def test_shuffle_matches_oracle(gpu, oracle, rows, cols):
     np.testing.assert_array_equal(out.cpu().numpy(), oracle.shuffle_int4_mfma(packed, rows, cols))
 
 
-# the reference-layout GEMM's shape list (tests/test_gpu_int4.py), every path:
-# X resident (one to four phases), K-split, the chunked and the four-tile
-# fallbacks, ragged row tiles, spare waves, group sizes 128..512
+# the reference-layout GEMM's shape lists (tests/test_gpu_int4.py): few rows
+# here, on the kernel for few weight rows (ragged row tiles, one to four tiles
+# of X, group sizes 128..512) and the K-split kernel at 28672 x 8192; more rows
+# than that kernel takes, for every other kernel, in LARGE_ROWS
 GEMM_SHAPES = [(3, 64, 256, 128), (17, 130, 2048, 256), (33, 48, 640, 128), (64, 16, 128, 128),
                (2, 250, 384, 128), (4, 1000, 1280, 256), (3, 4096, 4096, 128),
                (4, 7 * 16 * 3 + 5, 2048, 512), (4, 33, 32768, 128), (16, 48, 1024, 128),
@@ -84,21 +83,28 @@ GEMM_SHAPES = [(3, 64, 256, 128), (17, 130, 2048, 256), (33, 48, 640, 128), (64,
                (40, 113, 16384, 128), (17, 7, 256, 256), (63, 1, 512, 128), (26, 130, 1152, 128),
                (40, 200, 4096, 512), (64, 50, 24576, 128), (4, 28672, 8192, 128),
                (16, 28672, 8192, 128), (64, 28672, 8192, 128),
-               # the reference layout's pair form: one and three pairs per wave,
-               # K at its limit for M <= 16; past its limit for M <= 32
+               # K a multiple of 1024: whole pairs of T-blocks
                (3, 200, 1024, 128), (2, 77, 3072, 256), (8, 130, 12288, 128),
                (20, 60, 10240, 128)]
 
 
-def same_kernels(m, cols):
-    """Whether both layouts run the same GEMM kernel: the K-split kernel from
-    m = 9, and from m = 2 where the reference layout takes its pair form (K a
-    multiple of 1024, up to 12288); other m 2..8 shapes run the X-resident
-    kernel on the reference layout."""
-    return m >= 9 or (m >= 2 and cols % 1024 == 0 and cols <= 12288)
+def same_sums(m, rows, cols):
+    """Whether both layouts run the same products and sums, as the header
+    states: the kernel for few rows, and beyond it the K-split kernel (in
+    pairs of T-blocks on the reference layout only, with the same sums) or one
+    fallback on both, but not
+      * m 33..48 at K 12288: pairs through LDS, on the shuffled layout past the
+        LDS of the single form;
+      * m 2..8 where the pair form does not apply: X resident or chunked,
+        against the K-split kernel up to K 23040."""
+    if rows <= (16384 if m <= 16 else 8192):
+        return m >= 2
+    if m >= 9:
+        return not (33 <= m <= 48 and cols == 12288)
+    return (cols % 1024 == 0 and cols <= 12288) or cols > 23040
 
 
-@pytest.mark.parametrize("m,rows,cols,gs", GEMM_SHAPES)
+@pytest.mark.parametrize("m,rows,cols,gs", GEMM_SHAPES + [shape for shape, _ in LARGE_ROWS])
 def test_gemm_shuffled_equals_reference_layout(gpu, oracle, m, rows, cols, gs):
     torch = gpu
     packed, scales, zeros = make_int4(rows, cols, gs, seed=m * 1000 + rows)
@@ -107,7 +113,7 @@ def test_gemm_shuffled_equals_reference_layout(gpu, oracle, m, rows, cols, gs):
     ref = _gemm(torch, "kc_gemm_int4_bf16", dp, ds, dz, dx, m, rows, cols, gs)
     sh = _shuffle(torch, dp, rows, cols)
     y = _gemm(torch, "kc_gemm_int4_bf16_shuffled", sh, ds, dz, dx, m, rows, cols, gs)
-    if same_kernels(m, cols):
+    if same_sums(m, rows, cols):
         assert torch.equal(y.view(torch.int16), ref.view(torch.int16))
     else:
         truth = oracle.gemm_int4_bf16_f64(packed, scales, zeros.reshape(-1), xb, m, rows, cols, gs,
@@ -125,8 +131,10 @@ def test_gemm_shuffled_equals_reference_layout(gpu, oracle, m, rows, cols, gs):
                                           # (K 512 KW: 1536, 8192)
                                           (100, 1536, 128), (500, 8192, 128), (8192, 2048, 256),
                                           # K not a multiple of 1024 past N = 8192, or of 512:
-                                          # the X-resident kernel at M = 1
-                                          (9000, 1536, 128), (250, 1152, 128), (33, 640, 128)])
+                                          # the kernel for few rows at M = 1, past N = 16384
+                                          # the K-split kernel
+                                          (9000, 1536, 128), (250, 1152, 128), (33, 640, 128),
+                                          (16390, 1152, 128)])
 def test_gemv_shuffled_vs_oracle(gpu, oracle, rows, cols, gs):
     torch = gpu
     packed, scales, zeros = make_int4(rows, cols, gs, seed=rows * 7 + cols)
