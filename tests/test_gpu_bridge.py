@@ -137,37 +137,48 @@ def test_spans_emitted_with_reference_attributes(gpu):
         assert span.attributes[otel.CUDA_MS_ATTR] >= 0.0
 
 
-@pytest.mark.parametrize("rows,cols", [(3, 64), (5, 100), (257, 4104)])
-def test_outputs_on_reused_memory(gpu, rows, cols):
-    """Outputs are not cleared before a call: on memory that held NaN, and on
-    a side stream, every element is the one computed on fresh memory."""
+@pytest.mark.parametrize("rows,cols,gs", [(3, 64, 4), (5, 100, 4), (257, 4104, 4), (7, 96, 32), (130, 4128, 32),
+                                          (40, 4096, 128), (33, 5000, 40)])
+def test_outputs_on_reused_memory(gpu, monkeypatch, rows, cols, gs):
+    """Outputs are not cleared before a call, so every byte has to be written:
+    with each new output filled with 0x00, 0xFF (NaN) and 0x5A first, on a side
+    stream too, the results are the same."""
     torch = gpu
-    gs = 4
     g = torch.Generator(device="cuda").manual_seed(rows)
     packed = torch.randint(0, 256, (rows, cols // 2), dtype=torch.uint8, device="cuda", generator=g)
     zeros = torch.randint(0, 256, (rows, cols // gs), dtype=torch.uint8, device="cuda", generator=g)
     scales = torch.rand(rows, cols // gs, device="cuda", generator=g)
     x = torch.randn(rows, cols, device="cuda", generator=g)
+    s0 = x[0].abs() + 1.0
+    q0, qs0 = ops.fp8_quantize(x)
+    new, filled = torch.empty, []
 
-    def calls():
-        q, s = ops.fp8_quantize(x)
-        return [q, s, ops.fp8_dequantize(q, s, rows, cols), ops.smoothquant_scale(x, x[0].abs() + 1.0),
-                ops.int4_dequantize(packed, scales, zeros, rows, cols, gs),
-                ops.int4_gemv(packed, scales, zeros, x[0], rows, cols, gs)]
+    def results(fill):
+        def empty(*args, **kwargs):
+            t = new(*args, **kwargs)
+            if t.is_cuda and t.numel():
+                t.view(torch.uint8).fill_(fill)
+                filled.append(t.data_ptr())
+            return t
 
-    def poison():
-        for n in 2 * [rows * cols * 4, rows * cols, rows * 4]:
-            torch.full((n,), 255, dtype=torch.uint8, device="cuda")
+        monkeypatch.setattr(torch, "empty", empty)
+        out = [*ops.fp8_quantize(x), ops.fp8_quantize(x, per_token=False)[0],
+               ops.fp8_dequantize(q0, qs0, rows, cols), ops.fp8_dequantize(q0, qs0, rows, cols, per_token=False),
+               ops.smoothquant_scale(x, s0), ops.int4_dequantize(packed, scales, zeros, rows, cols, gs),
+               ops.int4_gemv(packed, scales, zeros, x[0], rows, cols, gs)]
+        monkeypatch.setattr(torch, "empty", new)
+        return out
 
-    first = [t.clone() for t in calls()]
+    first = results(0x00)
+    assert {t.data_ptr() for t in first} <= set(filled)
     torch.cuda.synchronize()
-    side = torch.cuda.Stream()
-    with torch.cuda.stream(side):
-        poison()
-        again = calls()
-    side.synchronize()
-    for a, b in zip(first, again):
-        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    for fill in (0xFF, 0x5A):
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            again = results(fill)
+        side.synchronize()
+        for a, b in zip(first, again):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     empty_q, empty_s = ops.fp8_quantize(torch.empty(rows, 0, device="cuda"))
     assert empty_q.shape == (rows, 0) and torch.equal(empty_s, torch.zeros(rows, device="cuda"))
 
