@@ -220,24 +220,23 @@ class _Span(contextlib.ContextDecorator):
     through the two generators of the recorded form, a 2.7 GHz Xeon).
     A span is entered once, as a generator's would be."""
 
-    __slots__ = ("_name", "_attrs", "_span", "_traced")
+    __slots__ = ("_args", "_span", "_traced")
 
-    def __init__(self, name: str, attrs: dict) -> None:
-        self._name = name
-        self._attrs = attrs
+    def __init__(self, *args: Any) -> None:  # name, attrs
+        self._args = args
 
     def _recreate_cm(self) -> "_Span":  # ContextDecorator: one span per call
-        return _Span(self._name, self._attrs)
+        return _Span(*self._args)
 
     def __enter__(self) -> Any:
-        name, attrs = self._name, self._attrs
-        del self._name, self._attrs  # AttributeError when entered again
-        if not _sinks and type(_get_tracer()) is LocalTracer:
-            self._traced = None
-            self._span = LocalSpan(name, recorded=False)
-            return self._span
-        self._traced = _traced_span(name, attrs)
-        return self._traced.__enter__()
+        name, attrs = self._args
+        del self._args  # AttributeError when entered again
+        if _sinks or type(_get_tracer()) is not LocalTracer:
+            self._traced = _traced_span(name, attrs)
+            return self._traced.__enter__()
+        self._traced = None
+        self._span = span = LocalSpan(name, False)
+        return span
 
     def __exit__(self, *exc: Any) -> Optional[bool]:
         if self._traced is not None:
