@@ -162,9 +162,11 @@ def _setup_prototypes(lib: ctypes.CDLL) -> None:
 def _stream() -> int:
     """The current torch stream of the current device (a hipStream_t) for the
     launchers: torch.cuda.current_stream().cuda_stream without the Stream
-    object around it (2.7 -> 0.1 us)."""
+    object around it (2.7 -> 0.1 us), by the function that torch's own compiled
+    code calls; through the Stream object where a torch has no such function."""
     import torch
-    return torch._C._cuda_getCurrentRawStream(-1)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return torch.cuda.current_stream().cuda_stream if raw is None else raw(-1)
 
 
 def _ptr(t) -> int:

@@ -162,6 +162,17 @@ def test_cpu_tensors_rejected():
         torch.ops.kernel_craft.fp8_quantize(x, True)
 
 
+def test_stream_lookup_without_the_raw_stream_function(monkeypatch):
+    """The current stream's handle comes from the Stream object where torch
+    does not export the raw lookup."""
+    import types
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 100 + device, raising=False)
+    assert ops._stream() == 99
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=7))
+    assert ops._stream() == 7
+
+
 def test_otel_local_spans_record_only_inside_a_recorder():
     """Without opentelemetry-api, spans are local records: attributes (and
     device timing) only while a recorded_spans() block collects them."""
