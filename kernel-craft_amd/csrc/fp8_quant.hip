@@ -521,7 +521,9 @@ __global__ __launch_bounds__(kThreads) void quant_tensor_f32_kernel(
 // Grid: one block per (row, kDequantCols-column tile); the row index is
 // uniform.  Two loads per thread before its first store: 8192 x 14336 97.4 us
 // against 110.2 with one and 108.5 with four (587 MB), 4096 x 4096 12.8 / 12.8 /
-// 13.2.  Nontemporal loads, plain stores, and 16-byte loads through LDS were
+// 13.2, each by itself on rotating buffers; right after the quantizer that
+// writes its codes it takes 4 us more (17.3 against 13.4 under the profiler, on
+// any number of buffers).  Nontemporal loads, plain stores, and 16-byte loads through LDS were
 // slower (16.4, 18.7 and 14.2 us at 4096 x 4096).
 // ---------------------------------------------------------------------------
 constexpr int kDequantTiles = 2;
@@ -994,9 +996,9 @@ int smoothquant_stats(const char* fn, const void* x, int64_t tokens, const void*
         // 1024 x 4096 fp32 9.5 -> 9.1 / 23.5 -> 22.7; level at 2 MB).  Larger ones
         // are streamed: kept, the quantizers gain 3 to 9 % at any size (2003 and
         // 14336 x 4096 70.9 -> 65.1), but the statistics by themselves, as a calibration
-        // runs them, lose 4 to 18 % at 38 to 60 MB (512 and 4096 x 4096 12.5 -> 13.0, on
-        // the same tensors 10.2 -> 11.0) and 6 to 10 % on new tensors beyond (28.0 ->
-        // 30.0; 28672 x 8192 85 -> 94).
+        // runs them, lose: 4 to 19 % on the same tensors at 38 to 83 MB (512 and 4096 x
+        // 4096 10.2 -> 11.0), 3 to 10 % on new ones at any size (134 MB 28.0 -> 30.0,
+        // 503 MB 85 -> 94).
         const bool keep = (tokens + outs) * cols * (BF16 ? 2 : 4) <= int64_t{28} << 20;
         const auto kernel = keep ? col_absmax2_kernel<BF16, true> : col_absmax2_kernel<BF16, false>;
         kernel<<<static_cast<unsigned>(blocks_x + blocks_w), kThreads, 0, stream>>>(

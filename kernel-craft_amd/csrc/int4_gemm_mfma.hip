@@ -23,7 +23,8 @@
 //     acc += s * C + c2 * sum_k X[m, k],   c2 = -s * (136 + z)
 // which removes the +128 encoding offset, the +8 of q ^ 8 and the zero point
 // exactly as the GEMV does.  Groups of 64 and 32 on 16-byte aligned operands
-// run gemm_int4_skinny_kernel, other shapes the GEMV per activation row.
+// run gemm_int4_skinny_kernel from M = 3 where it is expected to be faster;
+// those and the other shapes run the GEMV per activation row otherwise.
 //
 // Kernels, by M (kc_gemm_int4_bf16 at the bottom picks one), for more than 8192
 // weight rows (16384 at M <= 16); fewer run gemm_int4_skinny_kernel
@@ -43,7 +44,10 @@
 //             where gemm_int4_kslds_kernel's LDS does not fit;
 //   fallbacks gemm_int4_xres_kernel (M 2..16), gemm_int4_xbig_kernel
 //             (M 33..64) and gemm_int4_mfma_kernel (below) when the K-split
-//             kernels' coefficients do not fit in LDS (K above about 20000).
+//             kernels' coefficients do not fit in LDS (K above 23040), and
+//             the last at M 2..8 on the reference layout where the pair form
+//             does not apply and X has no phases that fit (T-blocks no
+//             multiple of 8, above all).
 //
 // gemm_int4_mfma_kernel work split.  A workgroup of NW waves owns
 // 16*RT*NW consecutive weight rows and the whole K; wave w owns row tiles
@@ -2069,7 +2073,8 @@ int gemm_int4(const char* fn, const uint8_t* d_packed, const float* d_scales,
         if (m == 1) {
             const int st = gemv_shuf(fn, d_packed, d_scales, d_zeros, d_x, d_y, rows, cols,
                                      kc::ilog2(group_size) - 7, stream);
-            if (st >= 0) return st;  // else the X-resident kernel below, at M = 1
+            // else, at M = 1: the few-rows kernel, past N = 16384 the K-split one
+            if (st >= 0) return st;
         }
     } else if (!fast || m == 1) {
         // Groups of 64 and 32 from M = 3 on the matrix cores, unless the GEMVs are
@@ -2122,7 +2127,7 @@ int gemm_int4(const char* fn, const uint8_t* d_packed, const float* d_scales,
     // else through registers (K 8192, N 28672, MI355X, reference layout:
     // M 16 / 32 / 48 / 64 in 26 / 31 / 38 / 47 us through LDS, 37 / 48 / 58 /
     // 69 us through registers, 41 / 77 / 95 / 101 us for the kernels below,
-    // which remain for shapes neither takes: K above about 20000, where the
+    // which remain for shapes neither takes: K above 23040, where the
     // coefficient stage does not fit in LDS, or operands of 4 GiB).
     if (m > kXresBestM || SHUF) {
         int st = -1;

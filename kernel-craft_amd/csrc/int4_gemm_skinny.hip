@@ -4,16 +4,21 @@
 //
 // gemm_int4_skinny_kernel: a workgroup of KW waves owns RT tiles of 16 weight
 // rows (RT 1 or 2) and all MT = ceil(M / 16) tiles of X.  Wave w takes the
-// pairs of T-blocks (128 k each) w, w + KW, ..., the next pair's weights and X
-// in registers on their way while one is multiplied; no barrier stands in the
-// loop, and the KW partial sums of every output meet in LDS in a fixed order.
+// pairs of T-blocks (128 k each) w, w + KW, ....  X runs one pair ahead: each
+// tile of the next pair's X is requested as soon as this pair's has been
+// multiplied; the weights have one set of registers, requested for the next
+// pair once both T-blocks of this one are multiplied (two to four sets were
+// slower: registers and occupancy).  No barrier stands in the loop, and the KW
+// partial sums of every output meet in LDS in a fixed order.
 // The K-split kernel's time hardly depends on N (K 14336: 47 us at M 16, 94 at
 // M 64, for 37 workgroups as for 74), this one's follows it:
 //   N 4096, K 14336: M 16 47.2 -> 15.0 us, M 32 68 -> 22.3, M 64 94 -> 38.4;
 //   N 6144, K 4096:  M 4 12.4 -> 7.3, M 16 12.5 -> 8.0, M 64 23.4 -> 17.6;
 //   N 14336, K 4096: M 12 12.5 -> 11.1.
-// Bound by the loads from the XCD's L2: every workgroup reads all of X (M 16,
-// N 4096: four times the weight bytes).
+// Bound by the loads from the XCD's L2, every workgroup reading all of X, and
+// by bringing X into operand order: M 16, N 4096, K 14336 reads 151 MB there for
+// 31 MB of weights and coefficients (10 TB/s), M 64 505 MB (13 TB/s), the matrix
+// cores 7 and 14 % busy.
 //
 // Loads.  One wave-wide load covers 8 whole 128-byte lines.  Weights of the
 // reference layout: load h of a pair takes rows 8 h .. 8 h + 7, lane (i, kb)
@@ -27,8 +32,9 @@
 // weights multiply.
 //
 // Groups of 64 and 32 (NG = 2, 4 groups per T-block): the operand lanes of the
-// other groups are zeroed, one product per group.  They took one GEMV per row
-// of X before.
+// other groups are zeroed, one product per group.  Two tokens, and some shapes
+// of three to six (gemvs_faster below), take one GEMV per row of X, as all did
+// before.
 #include <algorithm>
 #include <type_traits>
 
@@ -399,7 +405,9 @@ int gemm_skinny(const char* fn, const uint8_t* packed, const float* scales, cons
     }
     // Past these N the K-split kernel fills the chip (M 16, N 28672, K 4096:
     // 16.1 us there, 26.6 here; M 32, N 10240, K 4096 16.5 against 16.4; M 48
-    // 20.4 against 28.3).
+    // 20.4 against 28.3).  Up to them this kernel is the faster one at K 4096,
+    // 5120, 8192, 14336 and 20480, M 2 to 64, on both layouts: 4 to 8 % at the lines
+    // (M 16, N 16384, K 8192 22.4 -> 21.5 us; M 64, N 8192, K 8192 39.1 -> 29.7).
     if (N > (M <= 16 ? 4 : 2) * kOneTileRows) return -1;
     return by_tokens<1, SHUF>(fn, packed, scales, zeros, X, Y, M, N, K, kc::ilog2(group_size) - 7, stream);
 }
