@@ -518,33 +518,39 @@ __global__ __launch_bounds__(kThreads) void quant_tensor_f32_kernel(
 // ---------------------------------------------------------------------------
 // Dequantization (fp8_quant.cu:145-160): exact E4M3 decode
 // (v_cvt_pk_f32_fp8), times the row's (or the tensor's) scale.
-// Grid: one block per (row, kDequantCols-column tile); the row index is
-// uniform.  Two loads per thread before its first store: 8192 x 14336 97.4 us
-// against 110.2 with one and 108.5 with four (587 MB), 4096 x 4096 12.8 / 12.8 /
-// 13.2, each by itself on rotating buffers; right after the quantizer that
-// writes its codes it takes 4 us more (17.3 against 13.4 under the profiler, on
-// any number of buffers).  Nontemporal loads, plain stores, and 16-byte loads through LDS were
-// slower (16.4, 18.7 and 14.2 us at 4096 x 4096).
+// Grid: one block per (row, TILES x 1024 columns); the row index is uniform.
+//
+// One load per thread, or two before its first store, where the 1024-column
+// tiles of a row pair up and there are at least 4096 such blocks.  Two gain
+// where the row's last tile is part filled (4096 x 1032 7.0 -> 5.2 us, 4096 x
+// 3080 13.5 -> 11.5) and right after the quantizer that wrote the codes (4096 x
+// 4096 18.5 -> 17.3, 8192 x 14336 107 -> 95, under the profiler), and lose 2 to 4 %
+// elsewhere when they run by themselves (4096 x 4096 13.0 -> 13.3, 8192 x 14336 78.8
+// -> 81.6).  With an odd number of tiles half a block idles (4096 x 2052 8.8 ->
+// 10.9, 8192 x 2560 15.4 -> 18.4), and small grids lose what the second load
+// takes (64 x 4096 2.20 -> 2.36; after the quantizer 2.7 -> 3.2).  Four loads,
+// nontemporal loads, plain stores, and 16-byte loads through LDS were slower
+// (4096 x 4096).
 // ---------------------------------------------------------------------------
-constexpr int kDequantTiles = 2;
-constexpr int kDequantCols = kDequantTiles * 1024;
+constexpr int64_t kDequantPairBlocks = 4096;
 
+template <int TILES>
 __global__ __launch_bounds__(kThreads) void dequant_fp8_kernel(
     const int8_t* __restrict__ in, const float* __restrict__ scales, float* __restrict__ out,
     int64_t cols, int64_t tiles_per_row, bool per_token, bool vec) {
     const int64_t row = blockIdx.x / tiles_per_row;
     const int64_t tile = blockIdx.x - row * tiles_per_row;
     const float s = per_token ? scales[row] : scales[0];
-    const int64_t c0 = tile * kDequantCols + 4 * static_cast<int64_t>(threadIdx.x);
+    const int64_t c0 = tile * (TILES * 1024) + 4 * static_cast<int64_t>(threadIdx.x);
     const int8_t* src = in + row * cols;
     float* dst = out + row * cols;
     if (vec) {  // cols % 4 == 0
-        uint32_t q[kDequantTiles];
+        uint32_t q[TILES];
 #pragma unroll
-        for (int j = 0; j < kDequantTiles; ++j)
+        for (int j = 0; j < TILES; ++j)
             q[j] = *reinterpret_cast<const uint32_t*>(src + std::min(c0 + 1024 * j, cols - 4));
 #pragma unroll
-        for (int j = 0; j < kDequantTiles; ++j) {
+        for (int j = 0; j < TILES; ++j) {
             const int64_t c = c0 + 1024 * j;
             if (c >= cols) break;
             const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(q[j]), false);
@@ -554,7 +560,7 @@ __global__ __launch_bounds__(kThreads) void dequant_fp8_kernel(
         }
         return;
     }
-    for (int j = 0; j < kDequantTiles; ++j) {
+    for (int j = 0; j < TILES; ++j) {
         const int64_t c = c0 + 1024 * j;
         for (int64_t k = c; k < std::min(c + 4, cols); ++k) {
             const f32x2 a = __builtin_amdgcn_cvt_pk_f32_fp8(static_cast<int>(static_cast<uint8_t>(src[k])), false);
@@ -920,9 +926,12 @@ int dequant_fp8(const char* fn, const int8_t* in, const float* scales, float* ou
     if (rows == 0 || cols == 0) return KC_SUCCESS;
     int64_t tiles;
     unsigned grid;
-    if ((st = row_tiles(fn, rows, cols, kDequantCols, &tiles, &grid)) != KC_SUCCESS) return st;
+    const int64_t tiles1 = (cols + 1023) / 1024;
+    const bool pair = tiles1 % 2 == 0 && rows * (tiles1 / 2) >= kDequantPairBlocks;
+    if ((st = row_tiles(fn, rows, cols, pair ? 2048 : 1024, &tiles, &grid)) != KC_SUCCESS) return st;
     const bool vec = cols % 4 == 0 && kc::aligned(in, 4) && kc::aligned(out, 16);
-    dequant_fp8_kernel<<<grid, kThreads, 0, stream>>>(in, scales, out, cols, tiles, per_token, vec);
+    const auto kernel = pair ? dequant_fp8_kernel<2> : dequant_fp8_kernel<1>;
+    kernel<<<grid, kThreads, 0, stream>>>(in, scales, out, cols, tiles, per_token, vec);
     return kc::check_launch(fn);
 }
 

@@ -411,7 +411,11 @@ def test_e4m3_conversion_exhaustive(gpu, oracle):
 
 @pytest.mark.parametrize("per_token", [True, False])
 @pytest.mark.parametrize("rows,cols", [(1, 4), (3, 1020), (2, 1028), (3, 2048), (2, 2052), (5, 4100),
-                                       (7, 1001), (2, 2049)])
+                                       (7, 1001), (2, 2049),
+                                       # two loads per thread: an even number of
+                                       # 1024-column tiles and 4096 blocks
+                                       (4096, 1028), (4097, 2048), (4099, 1501), (2050, 3076), (2048, 4096),
+                                       (4096, 2052), (4095, 1028)])
 def test_dequant_column_tiles(gpu, oracle, rows, cols, per_token):
     """One and two 1024-column loads per thread, tiles cut at and beside their
     edges, and columns that are not a multiple of 4."""
