@@ -604,8 +604,8 @@ __global__ __launch_bounds__(kThreads) void dequant_int4_generic_kernel(
 }
 
 // 4 packed bytes -> 8 fp32 (two 16-byte stores) per thread; requires K % 8 == 0
-// and gs % 8 == 0 so the 8 outputs share one group.  For shapes that the
-// kernel below does not take.
+// and gs % 8 == 0 so the 8 outputs share one group.  For shapes and sizes that
+// the kernel below does not take.
 __global__ __launch_bounds__(kThreads) void dequant_int4_fast_kernel(
     const uint8_t* __restrict__ packed, const float* __restrict__ scales,
     const uint8_t* __restrict__ zeros, float* __restrict__ out, int64_t rows, int64_t cols,
@@ -644,6 +644,10 @@ __global__ __launch_bounds__(kThreads) void dequant_int4_fast_kernel(
 // 128, 71.4 us with two interleaved 16-byte stores per lane and a 64-bit
 // division per 8 weights -> 46.6 us here with U = 4 (266 MB; a fill of the 235 MB
 // written takes 30 us); U = 1 46.4, but 4096 x 4096 14.7 against 12.8.
+// From 288 workgroups' worth of chunks (2.4 M weights): 640 x 4096 5.5 -> 5.0 us,
+// 1024 x 4096 7.2 -> 5.1; below, the chain through LDS costs as much as it saves
+// or more (512 x 4096 4.8 against 5.1, 64 x 4096 2.7 against 3.2; 320 to 480 x 4096
+// 5 % either way) and the kernel above runs.
 template <int U>
 __global__ __launch_bounds__(kThreads) void dequant_int4_chunk_kernel(
     const uint8_t* __restrict__ packed, const float* __restrict__ scales,
@@ -902,10 +906,11 @@ int dequant_int4(const char* fn, const uint8_t* packed, const float* scales, con
     int st = check_int4_args(fn, packed, scales, zeros, packed, out, rows, cols, gs);
     if (st != KC_SUCCESS) return st;
     if (rows == 0 || cols == 0) return KC_SUCCESS;
+    constexpr int64_t kRun = kWavesPerBlock * kWave;
     const int64_t chunks = rows * (cols >> 5);
-    if (cols % 32 == 0 && gs % 32 == 0 && kc::aligned(packed, 16) && kc::aligned(out, 16) && chunks < INT32_MAX) {
+    if (cols % 32 == 0 && gs % 32 == 0 && kc::aligned(packed, 16) && kc::aligned(out, 16) &&
+        chunks >= 288 * kRun && chunks < INT32_MAX) {
         // four runs per wave where that leaves two workgroups per CU
-        constexpr int64_t kRun = kWavesPerBlock * kWave;
         const auto launch = [&](auto kernel, int64_t per_block) {
             kernel<<<static_cast<unsigned>((chunks + per_block - 1) / per_block), kThreads, 0, stream>>>(
                 packed, scales, zeros, out, static_cast<uint32_t>(chunks), static_cast<uint32_t>(cols >> 5),

@@ -138,7 +138,7 @@ def test_spans_emitted_with_reference_attributes(gpu):
 
 
 @pytest.mark.parametrize("rows,cols,gs", [(3, 64, 4), (5, 100, 4), (257, 4104, 4), (7, 96, 32), (130, 4128, 32),
-                                          (40, 4096, 128), (33, 5000, 40)])
+                                          (640, 4096, 128), (40, 4096, 128), (33, 5000, 40)])
 def test_outputs_on_reused_memory(gpu, monkeypatch, rows, cols, gs):
     """Outputs are not cleared before a call, so every byte has to be written:
     with each new output filled with 0x00, 0xFF (NaN) and 0x5A first, on a side

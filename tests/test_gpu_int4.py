@@ -127,12 +127,14 @@ def test_gemv_f32_shapes(gpu, oracle, rows, cols, gs):
     assert rel_l2(y, truth) < TOL_F32
 
 
-# Dequantization in runs of 64 chunks of 32 weights: one and four runs per
-# wave (four from 2^19 chunks), a last run cut anywhere, groups that are not a
-# power of two, one group per row; K and groups not multiples of 32 take the
-# other two kernels.
+# Dequantization in runs of 64 chunks of 32 weights from 73728 chunks on: one
+# and four runs per wave (four from 2^19 chunks), a last run cut anywhere, groups
+# that are not a power of two, one group per row; fewer chunks, and K and groups
+# not multiples of 32, take the other two kernels.
 @pytest.mark.parametrize("rows,cols,gs", [(1, 32, 32), (65, 32, 32), (3, 1056, 96), (129, 2080, 32),
                                           (4096, 4096, 128), (4097, 4128, 32), (2731, 6144, 6144),
+                                          (73728, 32, 32), (73729, 32, 32), (36863, 64, 32), (2235, 1056, 96),
+                                          (1137, 2080, 32), (577, 4096, 4096),
                                           (7, 1000, 8), (33, 1032, 24)])
 def test_dequant_runs_bit_exact(gpu, oracle, rows, cols, gs):
     packed, scales, zeros = make_int4(rows, cols, gs, seed=rows * 3 + cols)
