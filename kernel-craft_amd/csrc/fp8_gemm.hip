@@ -21,8 +21,9 @@
 // output is within 2^-10 sum_k |product| of the exact sum.  The scales are
 // applied once per output: (acc * sx) * sw.
 //
-// Decode batches (M <= 64) and grids of too few such tiles run the kernels of
-// fp8_gemm_small.hip, with the same products and scaling.
+// Decode batches (M <= 64, but for short K at many output columns) and grids of
+// too few such tiles run the kernels of fp8_gemm_small.hip, with the same
+// products and scaling.
 //
 // Tiling.  A 512-thread workgroup (8 waves) computes a 256 x 256 tile of Y;
 // wave w owns the 128 x 64 block (w / 4, w % 4) as 8 x 4 MFMA tiles of

@@ -247,6 +247,31 @@ int skinny(const char* fn, const int8_t* qx, const float* sx, const int8_t* qw, 
     return launch_skinny<MT, 4, 4, 2, YBF16>(fn, qx, sx, qw, sw, y, M, N, K, stream);
 }
 
+// Past N 28672 a short K leaves each of the many workgroups above little but its
+// start and its sum through LDS, and 256 x 256 tiles are faster again, the more so
+// the fuller their rounds of 256 tiles (65536 columns) are; K that is no multiple
+// of 128 costs the kernel above, whose loads then straddle cache lines, about 20 %
+// more than the large tiles.  M 49 to 64, bf16: N 40000 16.0 -> 12.9 us at K 256 and
+// level from 1024, N 64000 32.7 -> 27.5 at K 1024, 3 % at 2048, and with K 2064 to
+// 6160 15 to 20 %; N 90000 level from 1024.  Fewer tokens only where fp32 rows are
+// stored (M 48, N 64000, K 512 bf16 8 % faster here, fp32 7 % slower; M 33, N 40000, K 624
+// 22 % slower, M 16, N 64000, K 128 12 %).  N 28673 to 32768 at K 256 fp32, M 64 21 %.
+template <bool YBF16>
+bool large_tiles_at_short_k(int mt, int N, int K) {
+    constexpr int64_t kRound = 256 * 256;  // columns of a round of large tiles
+    if (N <= 28672) return false;
+    const bool whole = K % kBK == 0;
+    const int64_t fill = 100 * int64_t{N} / ((N + kRound - 1) / kRound * kRound);  // per cent
+    if (mt == 4) {
+        if (fill <= 50) return !YBF16 && K <= 512;
+        if (fill <= 70) return K <= (whole ? 1024 : 1600);
+        return !whole || K <= 2048;
+    }
+    if (YBF16 || fill <= 50) return false;
+    if (mt == 1) return K <= 128;
+    return K <= (whole ? 256 * mt - 128 : fill <= 70 ? 640 : 1600);
+}
+
 // ---------------------------------------------------------------------------
 // M > 64.  A workgroup computes a tile of 16 TM WGM x 16 TN WGN outputs with
 // KG groups of WGM x WGN waves; group g takes K steps g, g + KG, ... and the
@@ -583,6 +608,7 @@ bool gemm_small(const char* fn, const int8_t* qx, const float* sx, const int8_t*
     if (K > INT32_MAX / 256 || N > INT32_MAX / 2) return false;
     if (M <= kSkinnyM) {
         const int m = static_cast<int>(M), n = static_cast<int>(N), k = static_cast<int>(K);
+        if (large_tiles_at_short_k<YBF16>((m + 15) / 16, n, k)) return false;
         switch ((m + 15) / 16) {
             case 1: *status = skinny<1, YBF16>(fn, qx, sx, qw, sw, y, m, n, k, stream); break;
             case 2: *status = skinny<2, YBF16>(fn, qx, sx, qw, sw, y, m, n, k, stream); break;

@@ -136,7 +136,9 @@ def test_random_shapes_bit_exact(gpu, oracle, M, N, K):
 SMALL_GRIDS = [(1, 1, 16), (8, 15, 128), (9, 17, 144), (16, 33, 1040), (5, 40, 2048), (5, 41, 2064),
                (17, 4097, 272), (64, 4096, 1024), (64, 112, 4112), (1, 8200, 2064), (33, 8193, 144),
                (32, 16400, 400), (48, 16401, 272), (64, 16386, 528),
-               (33, 28672, 144), (64, 28671, 272), (48, 28673, 272), (64, 32001, 144)]
+               (33, 28672, 144), (64, 28671, 272), (48, 28673, 272), (64, 32001, 144),
+               # past it, where fp32 rows at short K run the 256 x 256 tiles
+               (5, 34001, 128), (17, 34001, 384), (48, 34001, 640), (48, 34001, 656), (64, 32768, 512)]
 SMALL_GRIDS += [(m, n, k) for m, n in ((65, 131), (200, 2704), (500, 2701), (1000, 2700), (1500, 3900))
                 for k in (16, 272, 640, 1168, 2048)]
 # K of two steps: two rounds of 256 x 256 tiles, not three of smaller ones
@@ -161,7 +163,9 @@ def test_small_grids_bit_exact(gpu, oracle, M, N, K):
 # of 4 (four columns per lane) and odd, and K of a partial step only, one whole
 # step, one and a tail, odd and even step counts.
 BIG_TILES = [(2945, 2696, 16), (2945, 2700, 272), (3071, 2689, 128), (3072, 2816, 144), (500, 16520, 640),
-             (512, 16516, 1040), (449, 16641, 400)]
+             (512, 16516, 1040), (449, 16641, 400),
+             # 49 to 64 tokens, short K, more columns than 28672
+             (64, 40001, 272), (49, 50008, 144), (50, 34000, 1024), (64, 50000, 2064)]
 
 
 @pytest.mark.parametrize("M,N,K", BIG_TILES)
@@ -180,6 +184,8 @@ def test_big_tiles_bit_exact(gpu, oracle, M, N, K):
 @pytest.mark.parametrize("M,N,K,kernel", [(m, n, k, "gemm_fp8_kernel<") for m, n, k in BIG_TILES + [(1500, 14340, 144)]] + [
     (64, 4096, 1024, "gemm_fp8_skinny_kernel<4, 1,"), (33, 8193, 144, "gemm_fp8_skinny_kernel<3, 4,"),
     (64, 28671, 272, "gemm_fp8_skinny_kernel<4, 7,"), (48, 28673, 272, "gemm_fp8_skinny_kernel<3, 4,"),
+    (64, 33000, 1040, "gemm_fp8_skinny_kernel<4, 4,"), (48, 34001, 656, "gemm_fp8_skinny_kernel<3, 4,"),
+    (64, 50000, 2176, "gemm_fp8_skinny_kernel<4, 4,"),
     (65, 131, 2048, "gemm_fp8_tile_kernel<2, 2, 1, 2,"), (200, 2704, 16, "gemm_fp8_tile_kernel<4, 2, 1, 2,"),
     (500, 2701, 16, "gemm_fp8_tile_kernel<4, 2, 1, 4,"), (1000, 2700, 2048, "gemm_fp8_tile_kernel<4, 2, 2, 4,"),
     (1500, 3900, 2048, "gemm_fp8_tile_kernel<4, 4, 4, 2,")])
