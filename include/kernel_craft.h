@@ -229,7 +229,8 @@ int kc_gemm_int4_bf16(const uint8_t* d_packed, const float* d_scales,
  *   kc_gemm_int4_bf16_shuffled: kc_gemm_int4_bf16 on the shuffled weights,
  *     each wave-wide load reading 1 KB of the layout.  Bit-identical results
  *     (the same products and sums) with rows up to 16384 at m 2..16 and up
- *     to 8192 at m 17..64 (cols up to 72704), and with more rows for m >= 9
+ *     to 8192 at m 17..64 (cols up to 72704; m 2..8 with rows past 4096 only
+ *     from cols 640, past 8192 from 1024), and with more rows for m >= 9
  *     except m 33..48 at cols == 12288, and for m 2..8 at cols a multiple of
  *     1024 up to 12288 or past 23040.  The other shapes run kernels of
  *     another summation order on the two layouts.  m == 1 runs a matrix-core

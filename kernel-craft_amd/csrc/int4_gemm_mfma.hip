@@ -28,7 +28,8 @@
 //
 // Kernels, by M (kc_gemm_int4_bf16 at the bottom picks one), for more than 8192
 // weight rows (16384 at M <= 16); fewer run gemm_int4_skinny_kernel
-// (int4_gemm_skinny.hip):
+// (int4_gemm_skinny.hip), but not M <= 8 at K < 1024 past 4096 or 8192 rows on the
+// reference layout:
 //   M 2..64   gemm_int4_kslds_kernel: K split over the four waves of a CU, X
 //             and the weights streamed into LDS by direct-to-LDS loads; on
 //             the reference layout at M <= 48 with K a multiple of 1024 the

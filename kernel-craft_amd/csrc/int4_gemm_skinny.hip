@@ -409,6 +409,12 @@ int gemm_skinny(const char* fn, const uint8_t* packed, const float* scales, cons
     // 5120, 8192, 14336 and 20480, M 2 to 64, on both layouts: 4 to 8 % at the lines
     // (M 16, N 16384, K 8192 22.4 -> 21.5 us; M 64, N 8192, K 8192 39.1 -> 29.7).
     if (N > (M <= 16 ? 4 : 2) * kOneTileRows) return -1;
+    // Up to 8 tokens on the reference layout at K below 1024 the waves have a
+    // pair of T-blocks at most, and one wave per row tile over all of K
+    // (gemm_int4_mfma_kernel) is faster from two row tiles on: M 4, K 512, N 8192
+    // 4.0 against 4.2 us, N 12000 4.1 against 5.0; K 640 and 896 3 to 6 % slower up
+    // to N 8192, 3 to 17 % faster past it; K 1152 10 to 32 % slower.
+    if (!SHUF && M <= 8 && K < 1024 && N > (K <= 512 ? 1 : 2) * kOneTileRows) return -1;
     return by_tokens<1, SHUF>(fn, packed, scales, zeros, X, Y, M, N, K, kc::ilog2(group_size) - 7, stream);
 }
 

@@ -457,8 +457,11 @@ LARGE_ROWS = [
     # four tiles of X resident
     ((40, 8200, 24576, 128), "gemm_int4_xbig_kernel<"),
     ((48, 8195, 23552, 256), "gemm_int4_xbig_kernel<"),
-    # chunks of K through LDS
+    # chunks of K through LDS, also few tokens at short K on fewer rows
     ((4, 16500, 1280, 256), "gemm_int4_mfma_kernel<1,"),
+    ((3, 4097, 512, 256), "gemm_int4_mfma_kernel<1,"),
+    ((8, 8193, 896, 128), "gemm_int4_mfma_kernel<1,"),
+    ((2, 16384, 128, 128), "gemm_int4_mfma_kernel<1,"),
     ((12, 16400, 24576, 128), "gemm_int4_mfma_kernel<1,"),
     ((32, 8200, 24576, 128), "gemm_int4_mfma_kernel<2,"),
     ((40, 8200, 24704, 128), "gemm_int4_mfma_kernel<3,"),
@@ -480,6 +483,10 @@ def test_gemm_large_rows(gpu, oracle, m, rows, cols, gs):
 @pytest.mark.parametrize("shape,kernel", LARGE_ROWS + [
     ((16, 16384, 640, 128), "gemm_int4_skinny_kernel<1, 2, 4, 1, false>"),
     ((16, 4096, 640, 128), "gemm_int4_skinny_kernel<1, 1, 8, 1, false>"),
+    ((8, 4096, 512, 128), "gemm_int4_skinny_kernel<1, 1, 8, 1, false>"),
+    ((8, 8192, 640, 128), "gemm_int4_skinny_kernel<1, 2, 8, 1, false>"),
+    ((8, 8193, 1024, 512), "gemm_int4_skinny_kernel<1, 2, 4, 1, false>"),
+    ((9, 16384, 512, 128), "gemm_int4_skinny_kernel<1, 2, 4, 1, false>"),
     ((64, 8192, 640, 128), "gemm_int4_skinny_kernel<4, 2, 4, 1, false>"),
     ((64, 8200, 256, 64), "gemm_int4_skinny_kernel<4, 2, 4, 2, false>"),
     ((3, 4100, 1152, 32), "gemm_int4_skinny_kernel<1, 2, 8, 4, false>")])

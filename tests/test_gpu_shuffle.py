@@ -96,9 +96,11 @@ def same_sums(m, rows, cols):
       * m 33..48 at K 12288: pairs through LDS, on the shuffled layout past the
         LDS of the single form;
       * m 2..8 where the pair form does not apply: X resident or chunked,
-        against the K-split kernel up to K 23040."""
+        against the K-split kernel up to K 23040;
+      * m 2..8 at short K past 4096 or 8192 rows, chunked on the reference
+        layout."""
     if rows <= (16384 if m <= 16 else 8192):
-        return m >= 2
+        return m >= 9 or (m >= 2 and not (cols < 1024 and rows > (4096 if cols <= 512 else 8192)))
     if m >= 9:
         return not (33 <= m <= 48 and cols == 12288)
     return (cols % 1024 == 0 and cols <= 12288) or cols > 23040
